@@ -9,12 +9,16 @@
 // side and the activation as the "B" side, so each lane's accumulators hold 4
 // consecutive output columns of one output row.
 //
-// Main loop (K a multiple of 256, at least 512): a persistent kernel, one
-// workgroup per CU, streaming K through two 64 KB LDS pair slots (128 bytes
-// of K for the 256 A rows and 256 B rows) filled by buffer_load ... lds
-// straight from memory, one load per MFMA; the last K steps of a tile already
-// load the next tile's first pairs (details at gemm_fp8_ring).  Other K (a
-// multiple of 16) use a register-staged loop with K step 128.
+// Main loop of large outputs (K a multiple of 256, at least 512): a persistent
+// kernel, one workgroup per CU, streaming K through two 64 KB LDS pair slots
+// (128 bytes of K for the 256 A rows and 256 B rows) filled by buffer_load ...
+// lds straight from memory, one load per MFMA; the last K steps of a tile
+// already load the next tile's first pairs (details at gemm_fp8_ring; 192- and
+// 128-row tiles too).  Outputs that large tiles would spread over too few CUs
+// (and every K that is a multiple of 128 only) take tiles of 64 x 64 to 128 x
+// 256 (gemm_fp8_small); plan_gemm picks the tile.  Other K (a multiple of 16)
+// use a register-staged loop with K step 128.  Every kernel but the last sums
+// K in the same order, so the tile does not change a result's bits.
 //
 // Epilogue: y = acc * (sa[m] * sb[n]) + bias[n], rounded to bf16, leaves
 // through a per-wave LDS staging area as 16-byte row chunks:
@@ -113,54 +117,24 @@ struct CTile {
   __device__ __forceinline__ uint16_t LDS_AS* row(int r) const { return part[r >> 6] + (r & 63) * BN; }
 };
 
-template <int EPI>
-FVSR_DEV void epilogue(const v16f (&acc)[4][4], const CTile& ct, int64_t m0, int64_t n0,
-                       int64_t M, int64_t N, const EpiArgs& ep, int wm, int wn, int lane) {
-  // Phase 1: acc[i][j][g*4+r] is row ml = wm*128 + j*32 + (lane&31), column
-  // nl = wn*128 + i*32 + g*8 + (lane>>5)*4 + r.  8-byte units are XOR-swizzled
-  // with the row so 32 lanes writing 32 rows do not share banks.
-  float sam[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int64_t mg = m0 + wm * 128 + j * 32 + (lane & 31);
-    sam[j] = ep.sa[ep.sa_row ? (mg < M ? mg : M - 1) : 0];
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int nl = wn * 128 + i * 32 + g * 8 + (lane >> 5) * 4;
-      float sbv[4], bv[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t ng = n0 + nl + r < N ? n0 + nl + r : N - 1;
-        sbv[r] = ep.sb[ep.sb_col ? ng : 0];
-        bv[r] = ep.bias ? bf2f(ep.bias[ng]) : 0.0f;
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int ml = wm * 128 + j * 32 + (lane & 31);
-        float y[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) y[r] = acc[i][j][g * 4 + r] * (sam[j] * sbv[r]) + bv[r];
-        const int unit = (nl >> 2) ^ (ml & 63);
-        *(u32x2_t LDS_AS*)(ct.row(ml) + unit * 4) =
-            u32x2_t{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
-      }
-    }
-  }
-  __syncthreads();
-
-  // Phase 2: 32 threads per 512-byte row, 16 bytes (8 columns) each.
-  const int cpos = threadIdx.x & 31;
+// Second half of the block-wide epilogue: the TM x TN bf16 tile staged in LDS
+// (row_of(r) points at row r; its 4-column unit u sits at u ^ (r % (TN / 4)))
+// leaves as 16-byte chunks, TN / 8 threads per row, with the row-max and
+// gate-add epilogues applied on the way.
+template <int EPI, int TM, int TN, class RowOf>
+FVSR_DEV void epi_rows(const RowOf& row_of, int64_t m0, int64_t n0, int64_t M, int64_t N,
+                       const EpiArgs& ep) {
+  static_assert(EPI != FVSR_EPI_ROWMAX || TN % 128 == 0, "row maxima are per 128 columns");
+  constexpr int kChunks = TN / 8, kMask = TN / 4 - 1;
+  const int cpos = threadIdx.x % kChunks;
   const int64_t slab0 = n0 / 128;
-  for (int rr = threadIdx.x >> 5; rr < BM; rr += kThreads / 32) {
+  for (int rr = threadIdx.x / kChunks; rr < TM; rr += kThreads / kChunks) {
     const int64_t m = m0 + rr;
     const int nl = cpos * 8;
     const int64_t n = n0 + nl;
-    const uint16_t LDS_AS* crow = ct.row(rr);
-    const u32x2_t lo = *(const u32x2_t LDS_AS*)(crow + (((nl >> 2) ^ (rr & 63)) * 4));
-    const u32x2_t hi = *(const u32x2_t LDS_AS*)(crow + ((((nl >> 2) + 1) ^ (rr & 63)) * 4));
+    const uint16_t LDS_AS* crow = row_of(rr);
+    const u32x2_t lo = *(const u32x2_t LDS_AS*)(crow + (((nl >> 2) ^ (rr & kMask)) * 4));
+    const u32x2_t hi = *(const u32x2_t LDS_AS*)(crow + ((((nl >> 2) + 1) ^ (rr & kMask)) * 4));
     u32x4_t v = {lo[0], lo[1], hi[0], hi[1]};
     float vmax = -__builtin_huge_valf();
     if (EPI == FVSR_EPI_ROWMAX) {
@@ -215,14 +189,57 @@ FVSR_DEV void epilogue(const v16f (&acc)[4][4], const CTile& ct, int64_t m0, int
   }
 }
 
+template <int EPI>
+FVSR_DEV void epilogue(const v16f (&acc)[4][4], const CTile& ct, int64_t m0, int64_t n0,
+                       int64_t M, int64_t N, const EpiArgs& ep, int wm, int wn, int lane) {
+  // Phase 1: acc[i][j][g*4+r] is row ml = wm*128 + j*32 + (lane&31), column
+  // nl = wn*128 + i*32 + g*8 + (lane>>5)*4 + r.  8-byte units are XOR-swizzled
+  // with the row so 32 lanes writing 32 rows do not share banks.
+  float sam[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int64_t mg = m0 + wm * 128 + j * 32 + (lane & 31);
+    sam[j] = ep.sa[ep.sa_row ? (mg < M ? mg : M - 1) : 0];
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int nl = wn * 128 + i * 32 + g * 8 + (lane >> 5) * 4;
+      float sbv[4], bv[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t ng = n0 + nl + r < N ? n0 + nl + r : N - 1;
+        sbv[r] = ep.sb[ep.sb_col ? ng : 0];
+        bv[r] = ep.bias ? bf2f(ep.bias[ng]) : 0.0f;
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int ml = wm * 128 + j * 32 + (lane & 31);
+        float y[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[r] = acc[i][j][g * 4 + r] * (sam[j] * sbv[r]) + bv[r];
+        const int unit = (nl >> 2) ^ (ml & 63);
+        *(u32x2_t LDS_AS*)(ct.row(ml) + unit * 4) =
+            u32x2_t{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
+      }
+    }
+  }
+  __syncthreads();
+
+  epi_rows<EPI, BM, BN>([&](int r) { return ct.row(r); }, m0, n0, M, N, ep);
+}
+
 // ---------------------------------------------------------------------------
-// Main loop, K % 64 == 0 and K >= 256: persistent direct-to-LDS ring.
+// Main loop, K % 256 == 0 and K >= 512: persistent direct-to-LDS ring.
 // ---------------------------------------------------------------------------
 // Tile shapes of the ring kernel: 256 output columns (B rows) by TM = 64 * MJ
 // output rows (A rows); each of the 4 waves owns TM / 2 rows (MJ blocks of
-// 32) by 128 columns (4 blocks).  MJ = 4 (256 x 256) everywhere except where
-// a single round of 128-row tiles covers the output that 256-row tiles would
-// leave mostly idle (C1: 4224 x 1536 is 102 tiles of 256 rows, 198 of 128).
+// 32) by 128 columns (4 blocks).  MJ = 4 (256 x 256) has the least LDS traffic
+// per MFMA; MJ = 3 and 2 are for outputs whose rounds they fill better (C1:
+// 4224 x 1536 is 102 tiles of 256 rows but 198 of 128, 22 -> 15.5 us; 7000 x
+// 1536 is 168 tiles of 256 rows but 222 of 192: K = 1536 20.9 -> 18.9 us,
+// K = 8960 87.7 -> 74.5 us).
 template <int MJ>
 struct Tile {
   static constexpr int TM = 64 * MJ;
@@ -697,7 +714,7 @@ template <int EPI, bool DIRECT, int MJ, bool TOUCH = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
 void gemm_fp8_ring(const uint8_t* __restrict__ A, int64_t lda, const uint8_t* __restrict__ B,
                    int64_t ldb, int64_t M, int64_t N, int64_t K, EpiArgs ep) {
-  static_assert(MJ == 4 || (MJ == 2 && DIRECT), "128-row tiles take the fast epilogue only");
+  static_assert(MJ == 4 || DIRECT, "128- and 192-row tiles take the fast epilogue only");
   constexpr int TM = Tile<MJ>::TM;
   __shared__ __attribute__((aligned(1024))) uint8_t pair0[Tile<MJ>::kPairBytes];
   __shared__ __attribute__((aligned(1024))) uint8_t pair1[Tile<MJ>::kPairBytes];
@@ -809,6 +826,230 @@ void gemm_fp8_ring(const uint8_t* __restrict__ A, int64_t lda, const uint8_t* __
 }
 
 // ---------------------------------------------------------------------------
+// Small outputs, K % 128 == 0: one tile per workgroup, S-slot LDS pipeline.
+// ---------------------------------------------------------------------------
+// What bounds it: the LDS.  A step's time follows its LDS bytes (fragment
+// reads, each operand row twice, plus the loads' writes) at 128 bytes per
+// clock: 64 x 64 48 KB, 64 x 128 72 KB, 128 x 128 96 KB, 128 x 256 144 KB
+// against measured 380, 620, 810 and 1240 clocks of a 128-byte K step; its
+// MFMAs take 128, 256, 512 and 1024.  Three or four slots cover the memory
+// latency (with two, 128 x 128 takes 47 us where four take 29, K = 8960).
+// Measured (graph-replayed, 256 x 256 or 128 x 256 ring -> here, us, N = 1536):
+// M = 512, K = 1536 14.0 -> 5.5; M = 2079 15.3 -> 11.3; K = 8960: M = 512 57.5
+// -> 16.2, M = 1152 59.1 -> 24.4, M = 3072 58.5 -> 45.5.
+// Scheduling of one step: MFMA q is preceded by its share of the NL loads and,
+// in the first half of the step, followed by its share of the ND fragment reads.
+template <bool LOADS, int NM, int NL, int ND, int Q>
+FVSR_DEV void small_slot() {
+  constexpr int NH = NM / 2;
+  if (LOADS) __builtin_amdgcn_sched_group_barrier(kSgVmemRead, NL * (Q + 1) / NM - NL * Q / NM, 0);
+  __builtin_amdgcn_sched_group_barrier(kSgMfma, 1, 0);
+  if (Q < NH)
+    __builtin_amdgcn_sched_group_barrier(kSgDsRead, ND * (Q + 1) / NH - ND * Q / NH, 0);
+}
+template <bool LOADS, int NM, int NL, int ND, int... Q>
+FVSR_DEV void small_sched(std::integer_sequence<int, Q...>) {
+  (small_slot<LOADS, NM, NL, ND, Q>(), ...);
+}
+
+// Tile of TM = 64 * MJ rows by TN = 64 * NI columns; each of the 4 waves owns
+// a 32 * MJ by 32 * NI quadrant.  K goes through S slots of 128 bytes (the
+// ring's slot layout) filled S - 1 slots ahead.
+template <int MJ, int NI, int S>
+struct SmallTile {
+  static constexpr int TM = 64 * MJ, TN = 64 * NI;
+  static constexpr int kSlotBytes = (TM + TN) * 128;
+  static constexpr int kLoadsA = TM / 32, kLoadsB = TN / 32;  // per wave and slot
+  static constexpr int kLoads = kLoadsA + kLoadsB;
+  static_assert(kSlotBytes >= TM * TN * 2 / S, "staging fits the slots");
+};
+
+template <int MJ, int NI, int S>
+struct SmallCtx {
+  i32x4_t ra, rb;
+  uint32_t oa[SmallTile<MJ, NI, S>::kLoadsA], ob[SmallTile<MJ, NI, S>::kLoadsB];
+  int wave, wm, wn, lane, KT;
+};
+
+template <int MJ, int NI, int S>
+FVSR_DEV void small_issue(uint8_t LDS_AS* slot, const SmallCtx<MJ, NI, S>& c, int kt) {
+  using T = SmallTile<MJ, NI, S>;
+#pragma unroll
+  for (int t = 0; t < T::kLoadsA; ++t)
+    fvsr_buffer_load_lds(c.ra, (void LDS_AS*)(slot + (c.wave * T::kLoadsA + t) * 1024), 16,
+                         __builtin_bit_cast(int, c.oa[t]), kt * 128, 0, 0);
+#pragma unroll
+  for (int t = 0; t < T::kLoadsB; ++t)
+    fvsr_buffer_load_lds(c.rb, (void LDS_AS*)(slot + T::TM * 128 + (c.wave * T::kLoadsB + t) * 1024),
+                         16, __builtin_bit_cast(int, c.ob[t]), kt * 128, 0, 0);
+}
+
+// MFMA fragments of one slot: both 64-byte halves of the wave's rows.
+template <int MJ, int NI>
+struct SmallFrags {
+  v8i a[2][MJ], b[2][NI];
+};
+
+template <int MJ, int NI, int S>
+FVSR_DEV void small_read(const uint8_t LDS_AS* slot, const SmallCtx<MJ, NI, S>& c,
+                         SmallFrags<MJ, NI>& f) {
+  const int ra = c.wm * (32 * MJ) + (c.lane & 31), rb = c.wn * (32 * NI) + (c.lane & 31);
+#pragma unroll
+  for (int hs = 0; hs < 2; ++hs) {
+    const int c0 = 4 * hs + 2 * (c.lane >> 5);
+#pragma unroll
+    for (int j = 0; j < MJ; ++j) f.a[hs][j] = read_frag(slot, ra + 32 * j, c0);
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      f.b[hs][i] = read_frag(slot + SmallTile<MJ, NI, S>::TM * 128, rb + 32 * i, c0);
+  }
+}
+
+// Step kt (128 bytes of K, whose fragments were read into `f` one step ago):
+// wait until this wave's loads of slot kt + 1 have landed and its reads of
+// slot kt are done, barrier (the same holds for every wave: slot kt + 1 is
+// whole and slot kt is free), stream step kt + S into slot kt (`cur`), read
+// slot kt + 1's fragments into `g` and run the step's MFMAs.  STEADY: step
+// kt + S exists, so the loads need no branch and are spread over the MFMAs.
+template <int MJ, int NI, int S, bool STEADY>
+FVSR_DEV void small_step(uint8_t LDS_AS* cur, const uint8_t LDS_AS* nxt,
+                         const SmallCtx<MJ, NI, S>& c, int kt, v16f (&acc)[NI][MJ],
+                         const SmallFrags<MJ, NI>& f, SmallFrags<MJ, NI>& g) {
+  using T = SmallTile<MJ, NI, S>;
+  __builtin_amdgcn_sched_barrier(0);
+  if (STEADY || kt + S <= c.KT)
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm((S - 2) * T::kLoads, 0));
+  else
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  if (STEADY || kt + S < c.KT) small_issue<MJ, NI, S>(cur, c, kt + S);
+  small_read<MJ, NI, S>(nxt, c, g);
+#pragma unroll
+  for (int hs = 0; hs < 2; ++hs)
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < MJ; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.b[hs][i], f.a[hs][j],
+                                                                     acc[i][j], 0, 0, 0, 0, 0, 0);
+  small_sched<STEADY, 2 * MJ * NI, T::kLoads, 4 * (MJ + NI)>(
+      std::make_integer_sequence<int, 2 * MJ * NI>{});
+}
+
+template <int EPI, int MJ, int NI, int S, int WPC>
+__global__ __launch_bounds__(kThreads, WPC) void gemm_fp8_small(
+    const uint8_t* __restrict__ A, int64_t lda, const uint8_t* __restrict__ B, int64_t ldb,
+    int64_t M, int64_t N, int64_t K, EpiArgs ep) {
+  using T = SmallTile<MJ, NI, S>;
+  static_assert(S >= 2 && S <= 6, "");
+  __shared__ __attribute__((aligned(1024))) uint8_t slot0[T::kSlotBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t slot1[T::kSlotBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t slot2[S > 2 ? T::kSlotBytes : 16];
+  __shared__ __attribute__((aligned(1024))) uint8_t slot3[S > 3 ? T::kSlotBytes : 16];
+  __shared__ __attribute__((aligned(1024))) uint8_t slot4[S > 4 ? T::kSlotBytes : 16];
+  __shared__ __attribute__((aligned(1024))) uint8_t slot5[S > 5 ? T::kSlotBytes : 16];
+  __shared__ __attribute__((aligned(16))) float prm[T::TM + 2 * T::TN];  // sa, sb, bias
+  uint8_t LDS_AS* sl[6] = {(uint8_t LDS_AS*)slot0, (uint8_t LDS_AS*)slot1, (uint8_t LDS_AS*)slot2,
+                           (uint8_t LDS_AS*)slot3, (uint8_t LDS_AS*)slot4, (uint8_t LDS_AS*)slot5};
+  const int tiles_m = (int)((M + T::TM - 1) / T::TM), tiles_n = (int)((N + T::TN - 1) / T::TN);
+  int tm, tn;
+  map_tile(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int64_t m0 = (int64_t)tm * T::TM, n0 = (int64_t)tn * T::TN;
+  SmallCtx<MJ, NI, S> c;
+  c.ra = make_rsrc(A);
+  c.rb = make_rsrc(B);
+  c.lane = threadIdx.x & 63;
+  c.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  c.wm = c.wave & 1;
+  c.wn = c.wave >> 1;
+  c.KT = (int)(K / 128);
+  const int rl = c.lane >> 3, cl = c.lane & 7;
+#pragma unroll
+  for (int t = 0; t < T::kLoadsA; ++t) {
+    const int r = c.wave * (T::TM / 4) + t * 8 + rl;
+    c.oa[t] = (uint32_t)((m0 + r < M ? m0 + r : M - 1) * lda + swz128(r, cl) * 16);
+  }
+#pragma unroll
+  for (int t = 0; t < T::kLoadsB; ++t) {
+    const int r = c.wave * (T::TN / 4) + t * 8 + rl;
+    c.ob[t] = (uint32_t)((n0 + r < N ? n0 + r : N - 1) * ldb + swz128(r, cl) * 16);
+  }
+  // The tile's epilogue parameters are fetched ahead of the operands (one row
+  // and one column per thread) and parked in LDS after the K loop.
+  static_assert(T::TM <= kThreads && T::TN <= kThreads, "one parameter per thread");
+  const int64_t pm = m0 + threadIdx.x < M ? m0 + threadIdx.x : M - 1;
+  const int64_t pn = n0 + threadIdx.x < N ? n0 + threadIdx.x : N - 1;
+  const float psa = ep.sa[ep.sa_row ? pm : 0], psb = ep.sb[ep.sb_col ? pn : 0];
+  const uint16_t pbias = ep.bias ? ep.bias[pn] : (uint16_t)0;
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    if (s < c.KT) small_issue<MJ, NI, S>(sl[s], c, s);
+  v16f acc[NI][MJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < MJ; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+  if (c.KT >= S)
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm((S - 1) * T::kLoads, 15));
+  else
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  SmallFrags<MJ, NI> f[2];
+  small_read<MJ, NI, S>(sl[0], c, f[0]);
+  constexpr int U = S % 2 ? 2 * S : S;  // steps per trip: slots and fragment sets both repeat
+  int kt = 0;
+  for (; kt + U + S <= c.KT; kt += U) {
+#pragma unroll
+    for (int s = 0; s < U; ++s)
+      small_step<MJ, NI, S, true>(sl[s % S], sl[(s + 1) % S], c, kt + s, acc, f[s % 2],
+                                  f[(s + 1) % 2]);
+  }
+  for (; kt < c.KT; kt += U) {
+#pragma unroll
+    for (int s = 0; s < U; ++s)
+      if (kt + s < c.KT)
+        small_step<MJ, NI, S, false>(sl[s % S], sl[(s + 1) % S], c, kt + s, acc, f[s % 2],
+                                     f[(s + 1) % 2]);
+  }
+
+  if (threadIdx.x < T::TM) prm[threadIdx.x] = psa;
+  if (threadIdx.x < T::TN) {
+    prm[T::TM + threadIdx.x] = psb;
+    prm[T::TM + T::TN + threadIdx.x] = bf2f(pbias);
+  }
+  __syncthreads();  // ... and every wave is done with the slots: the tile is staged in slot 0
+  uint16_t LDS_AS* ct = (uint16_t LDS_AS*)slot0;
+  const float LDS_AS* pl = (const float LDS_AS*)prm;
+  const int h = c.lane >> 5;
+#pragma unroll
+  for (int j = 0; j < MJ; ++j) {
+    const int ml = c.wm * (32 * MJ) + j * 32 + (c.lane & 31);
+    const float sam = pl[ml];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int nl = c.wn * (32 * NI) + i * 32 + g * 8 + h * 4;
+        const f32x4_t sb = *(const f32x4_t LDS_AS*)(pl + T::TM + nl);
+        const f32x4_t bv = *(const f32x4_t LDS_AS*)(pl + T::TM + T::TN + nl);
+        float y[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[r] = acc[i][j][g * 4 + r] * (sam * sb[r]) + bv[r];
+        *(u32x2_t LDS_AS*)(ct + ml * T::TN + (((nl >> 2) ^ (ml & (T::TN / 4 - 1))) * 4)) =
+            u32x2_t{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
+      }
+  }
+  __syncthreads();
+  epi_rows<EPI, T::TM, T::TN>([&](int r) { return (const uint16_t LDS_AS*)(ct + r * T::TN); }, m0,
+                              n0, M, N, ep);
+}
+
+// ---------------------------------------------------------------------------
 // Main loop, any K % 16 == 0: register-staged, K step 128, LDS double buffer.
 // ---------------------------------------------------------------------------
 constexpr int BKG = 128;
@@ -897,34 +1138,52 @@ void gemm_fp8_generic(const uint8_t* __restrict__ A, int64_t lda, const uint8_t*
   epilogue<EPI>(acc, ct, m0, n0, M, N, ep, wm, wn, lane);
 }
 
-enum class Path { kGeneric, kRing, kRingFast, kRingFast128 };
+// Kernels by tile: the register-staged fallback, the small-tile pipeline and
+// the persistent ring (kRing: general epilogue; kRing128 / 192 / 256: fast
+// epilogue).
+enum class Path { kGeneric, k64x64, k64x128, k128x128, k128x256, kRing, kRing128, kRing192,
+                  kRing256 };
 constexpr int64_t kTouchMinK = 4096;  // L2 prefetch of the pair loads from this K on
 
+struct GemmArgs {
+  const uint8_t* a;
+  int64_t lda;
+  const uint8_t* b;
+  int64_t ldb, M, N, K;
+  EpiArgs ep;
+};
+
+template <class Kernel>
+void start(Kernel kernel, unsigned grid, hipStream_t st, const GemmArgs& g) {
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), 0, st, g.a, g.lda, g.b, g.ldb, g.M, g.N,
+                     g.K, g.ep);
+}
+
 template <int EPI>
-void launch(Path path, unsigned grid, hipStream_t st, const uint8_t* a, int64_t lda,
-            const uint8_t* b, int64_t ldb, int64_t M, int64_t N, int64_t K, const EpiArgs& ep) {
-  if constexpr (EPI != FVSR_EPI_GATE_ADD) {  // gate-add keeps the general epilogue
-    if (path == Path::kRingFast) {
-      if (K >= kTouchMinK)
-        hipLaunchKernelGGL((gemm_fp8_ring<EPI, true, 4, true>), dim3(grid), dim3(kThreads), 0, st,
-                           a, lda, b, ldb, M, N, K, ep);
-      else
-        hipLaunchKernelGGL((gemm_fp8_ring<EPI, true, 4>), dim3(grid), dim3(kThreads), 0, st, a,
-                           lda, b, ldb, M, N, K, ep);
-      return;
-    }
-    if (path == Path::kRingFast128) {
-      hipLaunchKernelGGL((gemm_fp8_ring<EPI, true, 2>), dim3(grid), dim3(kThreads), 0, st, a, lda,
-                         b, ldb, M, N, K, ep);
-      return;
-    }
+void launch(Path path, unsigned grid, hipStream_t st, const GemmArgs& g) {
+  switch (path) {
+    case Path::kGeneric:
+      return start(gemm_fp8_generic<EPI>, grid, st, g);
+    case Path::kRing:
+      return start(gemm_fp8_ring<EPI, false, 4>, grid, st, g);
+    case Path::k64x128:
+      return start(gemm_fp8_small<EPI, 1, 2, 3, 2>, grid, st, g);
+    case Path::k128x128:
+      return start(gemm_fp8_small<EPI, 2, 2, 4, 1>, grid, st, g);
+    case Path::k128x256:
+      return start(gemm_fp8_small<EPI, 2, 4, 3, 1>, grid, st, g);
+    default:
+      break;
   }
-  if (path != Path::kGeneric)
-    hipLaunchKernelGGL((gemm_fp8_ring<EPI, false, 4>), dim3(grid), dim3(kThreads), 0, st, a, lda,
-                       b, ldb, M, N, K, ep);
-  else
-    hipLaunchKernelGGL(gemm_fp8_generic<EPI>, dim3(grid), dim3(kThreads), 0, st, a, lda, b, ldb,
-                       M, N, K, ep);
+  if constexpr (EPI != FVSR_EPI_ROWMAX) {  // row maxima need 128-column tiles
+    if (path == Path::k64x64) return start(gemm_fp8_small<EPI, 1, 1, 4, 2>, grid, st, g);
+  }
+  if constexpr (EPI != FVSR_EPI_GATE_ADD) {  // gate-add keeps the general epilogue
+    if (path == Path::kRing128) return start(gemm_fp8_ring<EPI, true, 2>, grid, st, g);
+    if (path == Path::kRing192) return start(gemm_fp8_ring<EPI, true, 3>, grid, st, g);
+    if (g.K >= kTouchMinK) return start(gemm_fp8_ring<EPI, true, 4, true>, grid, st, g);
+    return start(gemm_fp8_ring<EPI, true, 4>, grid, st, g);
+  }
 }
 
 // Workgroups of the persistent kernel: one per CU, rounded down to a multiple
@@ -936,6 +1195,77 @@ int64_t persistent_slots() {
       cus < 8)
     cus = 256;
   return (cus / 8) * 8;
+}
+
+struct Plan {
+  Path path;
+  unsigned grid;
+};
+
+int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// The kernel whose tiles finish first.  A CU works its tiles off one after the
+// other (or two side by side at half speed each), so a tile shape costs
+// rounds = ceil(tiles / CUs) times the clocks of one tile per 128 bytes of K:
+// what its LDS traffic takes at 128 bytes per clock (fragment reads plus the
+// loads' writes) for the tiles up to 128 x 256, its MFMAs (64 clocks each) for
+// the larger ones; 192 rows pay 8% for their larger share of loads (17% at
+// long K, where the 256-row kernel prefetches into L2).  Equal costs go to the
+// larger tile.  Over 24 shapes (M 100-18432, N 1536-8960, K 1536 and 8960) the
+// choice is within 4% of the fastest of the eight.
+// Where lines lie, both sides measured (us): M = 512 (N = K = 1536) 64 x 64
+// 5.5 against 64 x 128 7.1; M = 1152 8.5 / 8.2; M = 2079 128 x 128 11.3
+// against 64 x 128 11.7; M = 2800 ring 128 15.4 against 64 x 128 16.3; 12000
+// rows 192 against 256 32.7 / 35.4; 9000 rows 31.0 / 22.7.  At long K the
+// 128 x 256 tile of gemm_fp8_small (three slots, 4000 rows 50.5) replaces the
+// ring's (two, 59.4); at K = 1536 its longer start costs more (16.5 / 15.3).
+Plan plan_gemm(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int epilogue,
+               bool direct) {
+  struct Option {
+    Path path;
+    int rows, cols, cost, deep_cost;  // deep: K >= kTouchMinK
+  };
+  static constexpr Option kOptions[] = {
+      {Path::kRing256, 256, 256, 2048, 2048}, {Path::kRing, 256, 256, 2048, 2048},
+      {Path::kRing192, 192, 256, 1664, 1792}, {Path::kRing128, 128, 256, 1152, 1152},
+      {Path::k128x256, 128, 256, 1152, 1152}, {Path::k128x128, 128, 128, 768, 768},
+      {Path::k64x128, 64, 128, 576, 576},     {Path::k64x64, 64, 64, 384, 384},
+  };
+  // Every row offset of either operand within 32 bits; the ring takes K in
+  // pairs of 128 bytes, at least two of them.
+  const bool small = K % 128 == 0 && K > 0 && K < 0x7fffffffLL &&
+                     (M - 1) * lda + K <= 0xffffffffLL && (N - 1) * ldb + K <= 0xffffffffLL;
+  const bool ring = small && K % 256 == 0 && K >= 512;
+  // The fast epilogue needs whole column tiles.
+  const bool fast = ring && epilogue != FVSR_EPI_GATE_ADD && direct && N % BN == 0;
+  const bool deep = K >= kTouchMinK;
+  const int64_t slots = persistent_slots();
+  Plan best{Path::kGeneric, (unsigned)(cdiv(M, BM) * cdiv(N, BN))};
+  int64_t best_cost = INT64_MAX;
+  for (const Option& o : kOptions) {
+    bool ok = small;
+    if (o.path == Path::kRing) ok = ring && !fast;
+    if (o.path == Path::kRing256 || o.path == Path::kRing192) ok = fast;
+    if (o.path == Path::kRing128) ok = fast && !deep;
+    if (o.path == Path::k128x256) ok = small && (deep || !fast);
+    if (o.path == Path::k64x64) ok = small && epilogue != FVSR_EPI_ROWMAX;
+    if (!ok) continue;
+    const int64_t tiles = cdiv(M, o.rows) * cdiv(N, o.cols);
+    if (tiles > 0x7fffffff) continue;
+    const int64_t rounds = cdiv(tiles, slots), cost = rounds * (deep ? o.deep_cost : o.cost);
+    if (cost >= best_cost) continue;
+    best_cost = cost;
+    // Persistent kernels: the fewest workgroups (a multiple of the 8 XCDs)
+    // that still finish in the same number of rounds as one per CU, so no CU
+    // holds a round more than another (ffn0 2310 tiles: 232 workgroups of 10
+    // tiles and fewer instead of 256 of 9 or 10; qkv 240, o and ffn2 200): the
+    // critical path is unchanged and the idle CUs' power goes to the others'
+    // clock (ffn0 216 -> 210 us, o 40.8 -> 39.7 us on one box).
+    const bool persistent = o.path == Path::kRing || o.path == Path::kRing128 ||
+                            o.path == Path::kRing192 || o.path == Path::kRing256;
+    best = {o.path, (unsigned)(persistent && tiles > slots ? 8 * cdiv(tiles, 8 * rounds) : tiles)};
+  }
+  return best;
 }
 
 }  // namespace
@@ -967,42 +1297,17 @@ extern "C" int fvsr_fp8_gemm(const void* a, int64_t lda, const float* sa, int sa
              fvsr_gemm_amax_parts(N), (const uint16_t*)res, (const uint16_t*)gate,
              sa_mode == FVSR_SCALE_ROW, sb_col, vec_params, res_vec, direct};
   hipStream_t st = (hipStream_t)stream;
-  // Persistent ring: K a multiple of 256, at least 8 K steps, and every row
-  // offset of either operand within 32 bits.
-  const bool ring = K % 256 == 0 && K >= 512 && K < 0x7fffffffLL && (M - 1) * lda + K <= 0xffffffffLL &&
-                    (N - 1) * ldb + K <= 0xffffffffLL;
-  // The fast epilogue needs whole column tiles.  128-row tiles when one
-  // round of them covers the output (a 128-row tile takes about half as long
-  // as a 256-row one, and 256-row tiles would then be a partial round too).
-  const bool fast = ring && epilogue != FVSR_EPI_GATE_ADD && direct && N % BN == 0;
-  const int64_t slots = persistent_slots();
-  const int64_t tiles128 = ((M + 127) / 128) * ((N + BN - 1) / BN);
-  const Path path = !ring ? Path::kGeneric
-                    : !fast ? Path::kRing
-                    : tiles128 <= slots ? Path::kRingFast128 : Path::kRingFast;
-  const int64_t units = path == Path::kRingFast128 ? tiles128 : tiles;
-  // Persistent grid: the fewest workgroups (a multiple of the 8 XCDs) that
-  // still finish in the same number of rounds as one per CU, so no CU holds
-  // a round more than another (ffn0 2310 tiles: 232 workgroups of 10 tiles
-  // and fewer instead of 256 of 9 or 10; qkv 240, o and ffn2 200): the
-  // critical path is unchanged and the idle CUs' power goes to the others'
-  // clock (ffn0 216 -> 210 us, o 40.8 -> 39.7 us on one box).
-  int64_t grid64 = units;
-  if (ring && units > slots) {
-    const int64_t rounds = (units + slots - 1) / slots;
-    grid64 = 8 * ((units + 8 * rounds - 1) / (8 * rounds));
-  }
-  const unsigned grid = (unsigned)grid64;
-  const uint8_t *ap = (const uint8_t*)a, *bp = (const uint8_t*)b;
+  const GemmArgs g{(const uint8_t*)a, lda, (const uint8_t*)b, ldb, M, N, K, ep};
+  const Plan plan = plan_gemm(M, N, K, lda, ldb, epilogue, direct != 0);
   switch (epilogue) {
     case FVSR_EPI_BIAS:
-      launch<FVSR_EPI_BIAS>(path, grid, st, ap, lda, bp, ldb, M, N, K, ep);
+      launch<FVSR_EPI_BIAS>(plan.path, plan.grid, st, g);
       break;
     case FVSR_EPI_ROWMAX:
-      launch<FVSR_EPI_ROWMAX>(path, grid, st, ap, lda, bp, ldb, M, N, K, ep);
+      launch<FVSR_EPI_ROWMAX>(plan.path, plan.grid, st, g);
       break;
     default:
-      launch<FVSR_EPI_GATE_ADD>(path, grid, st, ap, lda, bp, ldb, M, N, K, ep);
+      launch<FVSR_EPI_GATE_ADD>(plan.path, plan.grid, st, g);
       break;
   }
   return fvsr_launch_status();
