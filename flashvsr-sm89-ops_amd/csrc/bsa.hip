@@ -22,6 +22,8 @@
 //                     16-lane group receives element i%4 of the 8 bytes
 //                     addressed by lane 4j + i/4, for j = 0..3).
 // Rows whose block list is empty produce zeros (lcsa/triton_lcsa.py:59-60).
+#include <algorithm>
+
 #include "common.h"
 
 namespace {
@@ -289,6 +291,18 @@ FVSR_DEV void bsa_step(uint8_t LDS_AS* cur, uint8_t LDS_AS* nxt, int it, const S
   }
 }
 
+// Floats of one piece's partial result: O^T of 128 queries x 128 dims, then
+// the queries' running maxima (log2 domain) and sums.
+constexpr int kPieceFloats = kBlk * kD + 2 * kBlk;
+
+// Stored token row of query position qpos of query block qb.
+template <int QM>
+FVSR_DEV int64_t query_token(int qb, int qpos, const int32_t* q_map, const WinGeo& geo) {
+  return QM == kMap   ? (int64_t)q_map[(int64_t)qb * kBlk + qpos]
+         : QM == kWin ? win_base(qb, geo) + win_slot(qpos, geo)
+                      : (int64_t)qb * kBlk + qpos;
+}
+
 // QM / KM: how query and key/value block positions become stored token rows
 // (kDirect, kMap or kWin, see above); the output rows are the query rows.
 // DENSE: every key block 0..maxk-1 is kept for every query block (the
@@ -305,17 +319,23 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
                     int64_t q_hs, int64_t kv_ts, int64_t kv_hs, int64_t o_ts, int64_t o_hs,
                     const int32_t* __restrict__ sel, const int32_t* __restrict__ cnt,
                     int64_t maxk, int NQ, float scale_log2, const int32_t* __restrict__ q_map,
-                    const int32_t* __restrict__ kv_map, WinGeo geo, int o_rows16) {
+                    const int32_t* __restrict__ kv_map, WinGeo geo, int o_rows16, int whole,
+                    int pieces, float* __restrict__ part) {
   __shared__ __attribute__((aligned(1024))) uint8_t stage0[kStage];
   __shared__ __attribute__((aligned(1024))) uint8_t stage1[kStage];
   uint8_t LDS_AS* st0 = (uint8_t LDS_AS*)stage0;
   uint8_t LDS_AS* st1 = (uint8_t LDS_AS*)stage1;
   // Workgroup ids are dispatched round robin over the 8 XCDs; give each XCD a
   // contiguous range of (head, query block) units so that neighbouring query
-  // blocks, whose local windows share most key blocks, share one L2.
-  const int total = (int)gridDim.x, per = total / 8, rem = total % 8;
-  const int xcd = blockIdx.x % 8, loc = blockIdx.x / 8;
-  const int unit = xcd < rem ? xcd * (per + 1) + loc : rem * (per + 1) + (xcd - rem) * per + loc;
+  // blocks, whose local windows share most key blocks, share one L2.  The
+  // first `whole` workgroups (a multiple of 8 if others follow) take a unit
+  // each; the rest one of the `pieces` parts of a later unit's kept blocks.
+  const bool is_piece = !DENSE && (int)blockIdx.x >= whole;
+  const int first = is_piece ? whole : 0;
+  const int total = is_piece ? (int)gridDim.x - whole : whole, per = total / 8, rem = total % 8;
+  const int xcd = (blockIdx.x - first) % 8, loc = (blockIdx.x - first) / 8;
+  const int slot = xcd < rem ? xcd * (per + 1) + loc : rem * (per + 1) + (xcd - rem) * per + loc;
+  const int unit = is_piece ? whole + slot / pieces : slot;
   constexpr int NW = DENSE ? 8 : 4;
   const int units_per_head = DENSE ? (NQ + 1) / 2 : NQ;
   const int h = unit / units_per_head, up = unit % units_per_head;
@@ -326,8 +346,7 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
   const int qb_raw = DENSE ? 2 * up + (wave >> 2) : up;
   const bool q_live = qb_raw < NQ;
   const int qb = q_live ? qb_raw : NQ - 1;
-  const int n = DENSE ? (int)maxk : cnt[(int64_t)h * NQ + qb];
-  const StepCtx c{2 * n, wave, lane, half, lane >> 4, lane & 15, scale_log2};
+  int n = DENSE ? (int)maxk : cnt[(int64_t)h * NQ + qb];
   const int32_t* blocks = DENSE ? nullptr : sel + ((int64_t)h * NQ + qb) * maxk;
   // The first two block ids load together with the count (the row holds maxk
   // entries; those past the count are unspecified and then unused), so the
@@ -337,6 +356,14 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
     b0 = blocks[0];
     b1 = blocks[maxk > 1 ? 1 : 0];
   }
+  if (is_piece) {
+    const int pc = slot % pieces, lo = n * pc / pieces;
+    n = n * (pc + 1) / pieces - lo;
+    blocks += lo;
+    if (n > 0) b0 = blocks[0];
+    if (n > 1) b1 = blocks[1];
+  }
+  const StepCtx c{2 * n, wave, lane, half, lane >> 4, lane & 15, scale_log2};
   Stream st;
   {
     const uint16_t* base = (wave >= NW / 2 ? v : k) + (int64_t)h * kv_hs;
@@ -366,9 +393,7 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
   // This lane's query (MFMA column) and its Q^T operand: d-step kk covers
   // dims kk*16 + half*8 .. +8.
   const int qpos = (wave & 3) * 32 + (lane & 31);
-  const int64_t qtok = QM == kMap   ? (int64_t)q_map[(int64_t)qb * kBlk + qpos]
-                       : QM == kWin ? win_base(qb, geo) + win_slot(qpos, geo)
-                                    : (int64_t)qb * kBlk + qpos;
+  const int64_t qtok = query_token<QM>(qb, qpos, q_map, geo);
   u32x4_t qf[8];
   {
     const uint16_t* qr = q + qtok * q_ts + (int64_t)h * q_hs;
@@ -396,6 +421,25 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
   const auto lsw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run),
                                                     false, false);
   const float l_tot = __uint_as_float(lsw[0]) + __uint_as_float(lsw[1]);
+  if (is_piece) {
+    // Unnormalised O^T as it lies in the registers (1 KB per store), then the
+    // queries' running maxima and sums; l = -1 marks a piece without blocks.
+    float* pp = part + (int64_t)slot * kPieceFloats;
+    if (n > 0) {
+#pragma unroll
+      for (int jd = 0; jd < 4; ++jd)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *(f32x4_t*)(pp + (((wave * 16) + jd * 4 + g) * 64 + lane) * 4) =
+              f32x4_t{acc[jd][g * 4 + 0], acc[jd][g * 4 + 1], acc[jd][g * 4 + 2],
+                      acc[jd][g * 4 + 3]};
+    }
+    if (half == 0) {
+      pp[kBlk * kD + wave * 32 + lane] = m_run;
+      pp[kBlk * kD + kBlk + wave * 32 + lane] = n > 0 ? l_tot : -1.0f;
+    }
+    return;
+  }
   const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
   if (DENSE) {
     __syncthreads();  // waves 4-7 stage through stage1, which the last step reads
@@ -440,6 +484,57 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
     const int64_t tr = __shfl(tq, r, 64);
     *(u32x4_t*)(o + tr * o_ts + (int64_t)h * o_hs + c16 * 8) = val;
   }
+}
+
+// Result of the split units: out = sum_s w_s O_s / sum_s w_s l_s over a unit's
+// pieces s, w_s = 2^(m_s - max m), in the pieces' register layout.  A workgroup
+// takes one 32-dim subtile (blockIdx.y) of one unit, a lane 16 bytes of each
+// of four 8-dim groups per piece.  Latency bound: every load (of up to P >=
+// `pieces` pieces; past the last one its values again, unused) is issued
+// before the first is needed.
+template <int QM, int P>
+__global__ __launch_bounds__(kThreads) void bsa_combine_kernel(
+    const float* __restrict__ part, int pieces, int whole, int NQ, uint16_t* __restrict__ o,
+    int64_t o_ts, int64_t o_hs, const int32_t* __restrict__ q_map, WinGeo geo) {
+  const int lane = threadIdx.x & 63, half = lane >> 5, wave = threadIdx.x >> 6;
+  const int unit = whole + (int)blockIdx.x, h = unit / NQ, qb = unit % NQ, jd = blockIdx.y;
+  const int qpos = wave * 32 + (lane & 31);
+  const float* p0 = part + (int64_t)blockIdx.x * pieces * kPieceFloats;
+  float m[P], l[P];
+  f32x4_t v[P][4];
+#pragma unroll
+  for (int s = 0; s < P; ++s) {
+    const float* pp = p0 + (int64_t)min(s, pieces - 1) * kPieceFloats;
+    m[s] = pp[kBlk * kD + qpos];
+    l[s] = pp[kBlk * kD + kBlk + qpos];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      v[s][g] = *(const f32x4_t*)(pp + ((wave * 16 + jd * 4 + g) * 64 + lane) * 4);
+  }
+  uint16_t* orow = o + query_token<QM>(qb, qpos, q_map, geo) * o_ts + (int64_t)h * o_hs;
+  __builtin_amdgcn_sched_barrier(0);
+  // A piece without blocks (l = -1) wrote no O and takes no part.
+  float mx = -__builtin_huge_valf();
+#pragma unroll
+  for (int s = 0; s < P; ++s)
+    if (l[s] != -1.0f) mx = fmaxf(mx, m[s]);
+  float lt = 0.0f, acc[16] = {};
+#pragma unroll
+  for (int s = 0; s < P; ++s) {
+    const bool any = s < pieces && l[s] != -1.0f;
+    const float w = any ? __builtin_amdgcn_exp2f(m[s] - mx) : 0.0f;
+    lt += any ? w * l[s] : 0.0f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[g * 4 + e] += any ? w * v[s][g][e] : 0.0f;
+  }
+  const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+    *(u32x2_t*)(orow + jd * 32 + g * 8 + half * 4) =
+        u32x2_t{pack_bf16x2(acc[g * 4 + 0] * inv, acc[g * 4 + 1] * inv),
+                pack_bf16x2(acc[g * 4 + 2] * inv, acc[g * 4 + 3] * inv)};
 }
 
 // One row of the block index per wave: the kept block ids ascending, then the
@@ -489,17 +584,67 @@ extern "C" int fvsr_block_index(const uint8_t* keep, int64_t H, int64_t NQ, int6
 
 namespace {
 
+// How a call's units are laid out: the first `whole` run as one workgroup
+// each, every later one as `pieces` workgroups over parts of its kept blocks
+// (partial results in the caller's workspace, then bsa_combine_kernel).
+//
+// Two workgroups of one CU work a block off in 2.0 us, one alone in 2.4: a CU
+// is nearly as fast with one.  So it is whole units per CU that must come out
+// even: 108 units (a 24 x 24 tile) leave 148 CUs idle, 792 (66 query blocks)
+// give 24 CUs a fourth unit while the others wait.  The units past a multiple
+// of the CU count are cut into pieces, as many as two per CU take at once, at
+// least four of the maxk index entries each (a piece costs its start, ~6 us, and 130
+// KB of partials written and read).  Measured (one piece -> split, us):
+// 12 x 9 x 36 blocks 75 -> 42, 12 x 4 x 16 38 -> 21, 4 x 36 x 72 129 -> 75,
+// 12 x 66 x 66 379 -> 348, 12 x 66 x 198 941 -> 883, 12 x 17 x 68 132 -> 107.
+// Not split, since it measured the same or slower: a last round more than
+// three quarters full (39 x 12 units, 102.8 whole, 101.7 in two; 83 x 12, 603 /
+// 606) and calls of six rounds and more (132 x 12, 564 / 572).
+struct Split {
+  int64_t whole, rest;
+  int pieces;
+  int64_t floats() const { return pieces > 1 ? rest * pieces * kPieceFloats : 0; }
+};
+
+Split plan_split(int64_t H, int64_t NQ, int64_t maxk) {
+  const int64_t units = H * NQ;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      cus < 8)
+    cus = 256;
+  cus &= ~7;
+  const Split plain{units, 0, 1};
+  const int64_t rest = units % cus;
+#ifdef FVSR_TUNE
+  if (g_split == 1) return plain;
+  if (g_split > 1) return Split{units - rest, rest, g_split};
+#endif
+  if (rest == 0 || units >= 6 * cus || (units > cus && 4 * rest > 3 * cus)) return plain;
+  const int64_t pieces = std::min({2 * cus / rest, maxk / 4, (int64_t)8});
+  return pieces > 1 ? Split{units - rest, rest, (int)pieces} : plain;
+}
+
 template <int QM, int KM, bool DENSE = false>
 void launch_bsa(const void* q, const void* k, const void* v, void* o, int64_t q_ts, int64_t q_hs,
                 int64_t kv_ts, int64_t kv_hs, int64_t o_ts, int64_t o_hs, const int32_t* sel,
                 const int32_t* cnt, int64_t maxk, int64_t H, int64_t NQ, float scale_log2,
-                const int32_t* q_map, const int32_t* kv_map, WinGeo geo, hipStream_t st) {
+                const int32_t* q_map, const int32_t* kv_map, WinGeo geo, hipStream_t st,
+                const Split* split = nullptr, float* part = nullptr) {
   const int64_t units = H * (DENSE ? (NQ + 1) / 2 : NQ);
-  hipLaunchKernelGGL((bsa_fwd_kernel<QM, KM, DENSE>), dim3((unsigned)units),
+  const Split sp = split && part ? *split : Split{units, 0, 1};
+  hipLaunchKernelGGL((bsa_fwd_kernel<QM, KM, DENSE>),
+                     dim3((unsigned)(sp.whole + sp.rest * sp.pieces)),
                      dim3(DENSE ? 2 * kThreads : kThreads), 0, st,
                      (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o,
                      q_ts, q_hs, kv_ts, kv_hs, o_ts, o_hs, sel, cnt, maxk, (int)NQ, scale_log2,
-                     q_map, kv_map, geo, (int)(aligned16(o) && (o_ts | o_hs) % 8 == 0));
+                     q_map, kv_map, geo, (int)(aligned16(o) && (o_ts | o_hs) % 8 == 0),
+                     (int)sp.whole, sp.pieces, part);
+  if (sp.rest == 0) return;
+  const auto combine = sp.pieces <= 4 ? bsa_combine_kernel<QM, 4> : bsa_combine_kernel<QM, 8>;
+  hipLaunchKernelGGL(combine, dim3((unsigned)sp.rest, 4), dim3(kThreads), 0, st,
+                     (const float*)part, sp.pieces, (int)sp.whole, (int)NQ, (uint16_t*)o, o_ts,
+                     o_hs, q_map, geo);
 }
 
 // Checks shared by both entry points.
@@ -519,29 +664,101 @@ int bsa_args_ok(const void* q, const void* k, const void* v, const void* o, int6
 
 }  // namespace
 
+extern "C" int64_t fvsr_bsa_workspace_floats(int64_t H, int64_t NQ, int64_t maxk) {
+  if (H <= 0 || NQ <= 0 || maxk <= 0 || H * NQ > 0x7fffffff) return 0;
+  return plan_split(H, NQ, maxk).floats();
+}
+
+namespace {
+
+// The split of a call given a workspace: none without one.
+int split_for(int64_t H, int64_t NQ, int64_t maxk, const float* ws, int64_t ws_floats, Split& sp) {
+  sp = Split{H * NQ, 0, 1};
+  if (!ws) return FVSR_OK;
+  sp = plan_split(H, NQ, maxk);
+  if (ws_floats < sp.floats()) return FVSR_EWORKSPACE;
+  return ((uintptr_t)ws & 15) ? FVSR_EUNSUPPORTED : FVSR_OK;
+}
+
+}  // namespace
+
+extern "C" int fvsr_bsa_fwd_ws(const void* q, const void* k, const void* v, void* o,
+                               int64_t q_tok_stride, int64_t q_head_stride, int64_t kv_tok_stride,
+                               int64_t kv_head_stride, int64_t o_tok_stride, int64_t o_head_stride,
+                               const int32_t* sel, const int32_t* cnt, int64_t maxk, int64_t H,
+                               int64_t NQ, int64_t NK, int64_t head_dim, float sm_scale,
+                               const int32_t* q_map, const int32_t* kv_map, float* workspace,
+                               int64_t workspace_floats, void* stream) {
+  if (H < 0 || NQ < 0 || NK < 0 || maxk < 0) return FVSR_EINVAL;
+  if (H * NQ == 0) return FVSR_OK;
+  int rc = bsa_args_ok(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride, kv_head_stride,
+                       o_tok_stride, o_head_stride, sel, cnt, head_dim, H, NQ);
+  if (rc != FVSR_OK) return rc;
+  if ((q_map == nullptr) != (kv_map == nullptr)) return FVSR_EUNSUPPORTED;
+  Split sp;
+  rc = split_for(H, NQ, maxk, workspace, workspace_floats, sp);
+  if (rc != FVSR_OK) return rc;
+  const float scale_log2 = sm_scale * 1.4426950408889634f;
+  const WinGeo geo{0, 0, 1, 1};
+  if (q_map)
+    launch_bsa<kMap, kMap>(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride,
+                           kv_head_stride, o_tok_stride, o_head_stride, sel, cnt, maxk, H, NQ,
+                           scale_log2, q_map, kv_map, geo, (hipStream_t)stream, &sp, workspace);
+  else
+    launch_bsa<kDirect, kDirect>(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride,
+                                 kv_head_stride, o_tok_stride, o_head_stride, sel, cnt, maxk, H,
+                                 NQ, scale_log2, nullptr, nullptr, geo, (hipStream_t)stream, &sp,
+                                 workspace);
+  return fvsr_launch_status();
+}
+
 extern "C" int fvsr_bsa_fwd(const void* q, const void* k, const void* v, void* o,
                             int64_t q_tok_stride, int64_t q_head_stride, int64_t kv_tok_stride,
                             int64_t kv_head_stride, int64_t o_tok_stride, int64_t o_head_stride,
                             const int32_t* sel, const int32_t* cnt, int64_t maxk, int64_t H,
                             int64_t NQ, int64_t NK, int64_t head_dim, float sm_scale,
                             const int32_t* q_map, const int32_t* kv_map, void* stream) {
-  if (H < 0 || NQ < 0 || NK < 0 || maxk < 0) return FVSR_EINVAL;
+  return fvsr_bsa_fwd_ws(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride, kv_head_stride,
+                         o_tok_stride, o_head_stride, sel, cnt, maxk, H, NQ, NK, head_dim,
+                         sm_scale, q_map, kv_map, nullptr, 0, stream);
+}
+
+extern "C" int fvsr_bsa_fwd_window_ws(const void* q, const void* k, const void* v, void* o,
+                                      int64_t q_tok_stride, int64_t q_head_stride,
+                                      int64_t kv_tok_stride, int64_t kv_head_stride,
+                                      int64_t o_tok_stride, int64_t o_head_stride,
+                                      const int32_t* sel, const int32_t* cnt, int64_t maxk,
+                                      int64_t H, int64_t NQ, int64_t NK, int64_t head_dim,
+                                      float sm_scale, int64_t frames, int64_t height,
+                                      int64_t width, int kv_raster, float* workspace,
+                                      int64_t workspace_floats, void* stream) {
+  if (H < 0 || NQ < 0 || NK < 0 || maxk < 0 || frames < 0 || height < 0 || width < 0)
+    return FVSR_EINVAL;
+  if (frames % 2 || height % 8 || width % 8) return FVSR_EINVAL;
+  if (frames * height * width != NQ * kBlk) return FVSR_EINVAL;
+  if (kv_raster && NK != NQ) return FVSR_EINVAL;
   if (H * NQ == 0) return FVSR_OK;
-  const int rc = bsa_args_ok(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride,
-                             kv_head_stride, o_tok_stride, o_head_stride, sel, cnt, head_dim, H,
-                             NQ);
+  int rc = bsa_args_ok(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride, kv_head_stride,
+                       o_tok_stride, o_head_stride, sel, cnt, head_dim, H, NQ);
   if (rc != FVSR_OK) return rc;
-  if ((q_map == nullptr) != (kv_map == nullptr)) return FVSR_EUNSUPPORTED;
+  // In-window byte offsets of the K/V stream are 32-bit: two frames of rows.
+  const int64_t hw = height * width;
+  if (kv_raster && 2 * hw * kv_tok_stride * 2 > 0xffffffffLL) return FVSR_EUNSUPPORTED;
+  if (hw > 0x3fffffff) return FVSR_EUNSUPPORTED;
+  Split sp;
+  rc = split_for(H, NQ, maxk, workspace, workspace_floats, sp);
+  if (rc != FVSR_OK) return rc;
   const float scale_log2 = sm_scale * 1.4426950408889634f;
-  const WinGeo geo{0, 0, 1, 1};
-  if (q_map)
-    launch_bsa<kMap, kMap>(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride,
-                           kv_head_stride, o_tok_stride, o_head_stride, sel, cnt, maxk, H, NQ,
-                           scale_log2, q_map, kv_map, geo, (hipStream_t)stream);
+  const WinGeo geo{(int)width, (int)hw, (int)(width / 8), (int)((height / 8) * (width / 8))};
+  if (kv_raster)
+    launch_bsa<kWin, kWin>(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride, kv_head_stride,
+                           o_tok_stride, o_head_stride, sel, cnt, maxk, H, NQ, scale_log2,
+                           nullptr, nullptr, geo, (hipStream_t)stream, &sp, workspace);
   else
-    launch_bsa<kDirect, kDirect>(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride,
-                                 kv_head_stride, o_tok_stride, o_head_stride, sel, cnt, maxk, H,
-                                 NQ, scale_log2, nullptr, nullptr, geo, (hipStream_t)stream);
+    launch_bsa<kWin, kDirect>(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride,
+                              kv_head_stride, o_tok_stride, o_head_stride, sel, cnt, maxk, H, NQ,
+                              scale_log2, nullptr, nullptr, geo, (hipStream_t)stream, &sp,
+                              workspace);
   return fvsr_launch_status();
 }
 
@@ -553,31 +770,10 @@ extern "C" int fvsr_bsa_fwd_window(const void* q, const void* k, const void* v, 
                                    int64_t H, int64_t NQ, int64_t NK, int64_t head_dim,
                                    float sm_scale, int64_t frames, int64_t height, int64_t width,
                                    int kv_raster, void* stream) {
-  if (H < 0 || NQ < 0 || NK < 0 || maxk < 0 || frames < 0 || height < 0 || width < 0)
-    return FVSR_EINVAL;
-  if (frames % 2 || height % 8 || width % 8) return FVSR_EINVAL;
-  if (frames * height * width != NQ * kBlk) return FVSR_EINVAL;
-  if (kv_raster && NK != NQ) return FVSR_EINVAL;
-  if (H * NQ == 0) return FVSR_OK;
-  const int rc = bsa_args_ok(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride,
-                             kv_head_stride, o_tok_stride, o_head_stride, sel, cnt, head_dim, H,
-                             NQ);
-  if (rc != FVSR_OK) return rc;
-  // In-window byte offsets of the K/V stream are 32-bit: two frames of rows.
-  const int64_t hw = height * width;
-  if (kv_raster && 2 * hw * kv_tok_stride * 2 > 0xffffffffLL) return FVSR_EUNSUPPORTED;
-  if (hw > 0x3fffffff) return FVSR_EUNSUPPORTED;
-  const float scale_log2 = sm_scale * 1.4426950408889634f;
-  const WinGeo geo{(int)width, (int)hw, (int)(width / 8), (int)((height / 8) * (width / 8))};
-  if (kv_raster)
-    launch_bsa<kWin, kWin>(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride, kv_head_stride,
-                           o_tok_stride, o_head_stride, sel, cnt, maxk, H, NQ, scale_log2,
-                           nullptr, nullptr, geo, (hipStream_t)stream);
-  else
-    launch_bsa<kWin, kDirect>(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride,
-                              kv_head_stride, o_tok_stride, o_head_stride, sel, cnt, maxk, H, NQ,
-                              scale_log2, nullptr, nullptr, geo, (hipStream_t)stream);
-  return fvsr_launch_status();
+  return fvsr_bsa_fwd_window_ws(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride,
+                                kv_head_stride, o_tok_stride, o_head_stride, sel, cnt, maxk, H, NQ,
+                                NK, head_dim, sm_scale, frames, height, width, kv_raster, nullptr,
+                                0, stream);
 }
 
 extern "C" int fvsr_attn_dense(const void* q, const void* k, const void* v, void* o,

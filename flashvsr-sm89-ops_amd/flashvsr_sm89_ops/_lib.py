@@ -67,6 +67,12 @@ _SIGS = {
                                _I64, _I64, _I64, _P, _P, _P, _P, _I64, _P], _I),
     "fvsr_bsa_fwd": ([_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _I64, _I64,
                       _I64, _I64, _I64, _F, _P, _P, _P], _I),
+    "fvsr_bsa_workspace_floats": ([_I64, _I64, _I64], _I64),
+    "fvsr_bsa_fwd_ws": ([_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _I64, _I64,
+                         _I64, _I64, _I64, _F, _P, _P, _P, _I64, _P], _I),
+    "fvsr_bsa_fwd_window_ws": ([_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _I64,
+                                _I64, _I64, _I64, _I64, _F, _I64, _I64, _I64, _I, _P, _I64, _P],
+                               _I),
     "fvsr_attn_dense": ([_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
                          _I64, _F, _P], _I),
     "fvsr_bsa_fwd_window": ([_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _I64,

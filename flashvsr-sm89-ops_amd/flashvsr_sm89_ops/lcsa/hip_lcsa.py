@@ -127,16 +127,19 @@ def block_sparse_attention_strided(q, k, v, keep, sm_scale=None, *, heads: int, 
         raise ValueError("out is required")
     _lib.require_dtype(out, torch.bfloat16, "out")
     o_strides = o_strides or q_strides
+    # Room for the partial results of units split over several workgroups.
+    ws_n = int(_lib.lib().fvsr_bsa_workspace_floats(H, NQ, maxk))
+    ws = torch.empty(ws_n, dtype=torch.float32, device=q.device) if ws_n else None
     if window is not None:
         _check_extent(q, NQ * BLOCK, *q_strides, heads, head_dim, "q")
         _check_extent(out, NQ * BLOCK, *o_strides, heads, head_dim, "out")
         _check_extent(k, NK * BLOCK, *kv_strides, heads, head_dim, "k")
         _check_extent(v, NK * BLOCK, *kv_strides, heads, head_dim, "v")
-        rc = _lib.lib().fvsr_bsa_fwd_window(
+        rc = _lib.lib().fvsr_bsa_fwd_window_ws(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
             q_strides[0], q_strides[1], kv_strides[0], kv_strides[1], o_strides[0], o_strides[1],
             sel.data_ptr(), cnt.data_ptr(), maxk, H, NQ, NK, head_dim, float(sm_scale),
-            frames, height, width, int(bool(kv_raster)), _lib.stream(q))
+            frames, height, width, int(bool(kv_raster)), _lib.ptr(ws), ws_n, _lib.stream(q))
         _lib.check(rc, "block_sparse_attention")
         return out
     if (q_map is None) != (kv_map is None):
@@ -152,11 +155,11 @@ def block_sparse_attention_strided(q, k, v, keep, sm_scale=None, *, heads: int, 
             if not m.is_contiguous() or m.numel() < want:
                 raise ValueError(f"{n} must be contiguous with at least {want} entries, "
                                  f"got {m.numel()}")
-    rc = _lib.lib().fvsr_bsa_fwd(
+    rc = _lib.lib().fvsr_bsa_fwd_ws(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
         q_strides[0], q_strides[1], kv_strides[0], kv_strides[1], o_strides[0], o_strides[1],
         sel.data_ptr(), cnt.data_ptr(), maxk, H, NQ, NK, head_dim, float(sm_scale),
-        _lib.ptr(q_map), _lib.ptr(kv_map), _lib.stream(q))
+        _lib.ptr(q_map), _lib.ptr(kv_map), _lib.ptr(ws), ws_n, _lib.stream(q))
     _lib.check(rc, "block_sparse_attention")
     return out
 

@@ -361,6 +361,34 @@ int fvsr_bsa_fwd_window(const void* q, const void* k, const void* v, void* o,
                         int64_t height, int64_t width, int kv_raster, void* stream);
 
 /*
+ * fvsr_bsa_fwd and fvsr_bsa_fwd_window with room for partial results.  Calls
+ * whose (head, query block) units do not fill the GPU evenly run some units as
+ * several workgroups over parts of their kept blocks, each writing an fp32
+ * partial result to `workspace`, and one more launch combines them.
+ *   fvsr_bsa_workspace_floats  floats such a call needs (0: it splits nothing);
+ *                              depends on the sizes and the current device only
+ *   workspace   16-byte aligned, at least that many floats (FVSR_EWORKSPACE
+ *               otherwise), used until the call's kernels have run; NULL: no
+ *               unit is split, exactly the call without _ws
+ * Splitting changes the order of the softmax sums, not their precision.
+ */
+int64_t fvsr_bsa_workspace_floats(int64_t H, int64_t NQ, int64_t maxk);
+int fvsr_bsa_fwd_ws(const void* q, const void* k, const void* v, void* o, int64_t q_tok_stride,
+                    int64_t q_head_stride, int64_t kv_tok_stride, int64_t kv_head_stride,
+                    int64_t o_tok_stride, int64_t o_head_stride, const int32_t* sel,
+                    const int32_t* cnt, int64_t maxk, int64_t H, int64_t NQ, int64_t NK,
+                    int64_t head_dim, float sm_scale, const int32_t* q_map,
+                    const int32_t* kv_map, float* workspace, int64_t workspace_floats,
+                    void* stream);
+int fvsr_bsa_fwd_window_ws(const void* q, const void* k, const void* v, void* o,
+                           int64_t q_tok_stride, int64_t q_head_stride, int64_t kv_tok_stride,
+                           int64_t kv_head_stride, int64_t o_tok_stride, int64_t o_head_stride,
+                           const int32_t* sel, const int32_t* cnt, int64_t maxk, int64_t H,
+                           int64_t NQ, int64_t NK, int64_t head_dim, float sm_scale,
+                           int64_t frames, int64_t height, int64_t width, int kv_raster,
+                           float* workspace, int64_t workspace_floats, void* stream);
+
+/*
  * Dense attention: fvsr_bsa_fwd with every key block kept for every query
  * block, for the cross-attention's softmax(Q K^T * sm_scale) V over the
  * prompt K/V cached by init_cross_kv (integrate.py:132-143; upstream
