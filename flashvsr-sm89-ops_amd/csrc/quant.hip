@@ -16,6 +16,7 @@
 // results, generated at build time from the operation sequence of
 // gelu_tanh_bf16 (csrc/gelu_table_gen.c), sit in every workgroup's LDS.
 #pragma clang fp contract(off)
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -55,6 +56,53 @@ FVSR_DEV float chunk_absmax(u32x4_t c) {
 FVSR_DEV float qscale(float amax) { return fmaxf(amax, 1e-12f) / 448.0f; }
 // The residual's copy of s, kept finite (s = inf when amax = inf).
 FVSR_DEV float qscale_fin(float s) { return fminf(s, 3.40282347e38f); }
+
+// Maximum over the workgroup's W waves of non-negative values (every load in
+// flight, into LDS too, has landed for all of them afterwards).
+template <int W>
+FVSR_DEV float block_max(float m, float* red) {
+  m = wave_max_abs(m);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  float r = red[0];
+#pragma unroll
+  for (int w = 1; w < W; ++w) r = fmaxf(r, red[w]);
+  return r;
+}
+
+// This thread's share (of T threads) of the largest of n partial maxima, 1 <= n
+// <= kMaxPartials: the loads are unconditional (past the end the last value
+// again), so they cost one memory latency together and not one each (the four
+// small passes of the per-tensor FFN at 8448 rows: 24 -> 20 us).
+template <int T>
+FVSR_DEV float max_partials(const float* __restrict__ part, int n) {
+  constexpr int U = (kMaxPartials + T - 1) / T;
+  float v[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int i = (int)threadIdx.x + u * T;
+    v[u] = part[i < n ? i : n - 1];
+  }
+  float m = v[0];
+#pragma unroll
+  for (int u = 1; u < U; ++u) m = fmaxf(m, v[u]);
+  return m;
+}
+
+// Calls f(chunk index, chunk) for the 16-byte chunks lane, lane + 64, ... of a
+// row of n chunks, U loads in flight (past the end the last chunk again).
+template <int U, class F>
+FVSR_DEV void for_chunks(const uint16_t* row, int64_t n, int lane, const F& f) {
+  for (int64_t c0 = lane; c0 < n; c0 += 64 * U) {
+    u32x4_t v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = *(const u32x4_t*)(row + clamp_chunk(c0 + 64 * u, n) * 8);
+#pragma unroll
+    for (int u = 0; u < U; ++u) f(c0 + 64 * u, v[u]);
+  }
+}
+constexpr int kChunkLoads = 3;  // a 1536-column row in one go
 
 // ---------------------------------------------------------------------------
 // Row mode, register resident: cols % 8 == 0, cols <= 512*VPL, 16-byte rows.
@@ -129,6 +177,22 @@ constexpr int kRowTabWaves = 8;
 // us against 80.4, and a pure row-streaming kernel at 80.3 us against 76.1.
 FVSR_DEV int64_t first_table_row() {
   return (int64_t)blockIdx.x + (int64_t)(threadIdx.x >> 6) * gridDim.x;
+}
+
+// Copy the table into LDS with direct loads, all 128 of 1 KB in flight at once:
+// a loop that loads 16 bytes per thread and stores them waits for memory on
+// each of its 16 trips (64 rows: 9.4 -> 5.6 us per token, 19.8 -> 11.7 per
+// tensor; 16896 rows 83.2 -> 81.8 and 133.6 -> 131.9).
+template <int WAVES>
+FVSR_DEV void load_table(uint16_t* tab) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint8_t* src = (const uint8_t*)kGeluTable + (threadIdx.x & 63) * 16;
+#pragma unroll
+  for (int c = 0; c < 128; c += WAVES)
+    if (c + wave < 128)
+      __builtin_amdgcn_global_load_lds(src + (c + wave) * 1024,
+                                       (__attribute__((address_space(3))) void*)(tab + (c + wave) * 512),
+                                       16, 0, 0);
 }
 
 // Load row `row` (chunks past the end of the row repeat its last chunk).
@@ -219,13 +283,9 @@ __global__ __launch_bounds__(kTabWaves * 64) void quant_tensor_gelu_table(
     const float* __restrict__ part, int nparts, uint8_t* __restrict__ codes,
     float* __restrict__ scale_out) {
   __shared__ __attribute__((aligned(16))) uint16_t tab[65536];
-  for (int i = threadIdx.x; i < 65536 / 8; i += kTabWaves * 64)
-    ((u32x4_t*)tab)[i] = ((const u32x4_t*)kGeluTable)[i];
-  const int lane = threadIdx.x & 63;
-  float m = 0.0f;
-  for (int i = lane; i < nparts; i += 64) m = fmaxf(m, part[i]);
-  const float amax = wave_max_abs(m);
-  __syncthreads();
+  __shared__ float red[kTabWaves];
+  load_table<kTabWaves>(tab);
+  const float amax = block_max<kTabWaves>(max_partials<kTabWaves * 64>(part, nparts), red);
   const float s = qscale(amax), r = 1.0f / s, sc = qscale_fin(s);
   if (blockIdx.x == 0 && threadIdx.x == 0) scale_out[0] = act_scale(amax);
   const int nchunk = (int)(cols >> 3);
@@ -245,8 +305,8 @@ __global__ __launch_bounds__(kTabWaves * 64) void amax_gelu_table(
     float* __restrict__ part) {
   __shared__ __attribute__((aligned(16))) uint16_t tab[65536];
   __shared__ float red[kTabWaves];
-  for (int i = threadIdx.x; i < 65536 / 8; i += kTabWaves * 64)
-    ((u32x4_t*)tab)[i] = ((const u32x4_t*)kGeluTable)[i];
+  load_table<kTabWaves>(tab);
+  __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   const int nchunk = (int)(cols >> 3);
   const int64_t stride = (int64_t)gridDim.x * kTabWaves;
@@ -260,14 +320,8 @@ __global__ __launch_bounds__(kTabWaves * 64) void amax_gelu_table(
       for (int i = 0; i < 4; ++i)
         m = max3_abs(m, bf2f(tab[v[j][i] & 0xffffu]), bf2f(tab[v[j][i] >> 16]));
   }
-  m = wave_max_abs(m);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float b = 0.0f;
-    for (int w = 0; w < kTabWaves; ++w) b = fmaxf(b, red[w]);
-    part[blockIdx.x] = b;
-  }
+  m = block_max<kTabWaves>(m, red);
+  if (threadIdx.x == 0) part[blockIdx.x] = m;
 }
 
 template <int VPL>
@@ -275,8 +329,8 @@ __global__ __launch_bounds__(kRowTabWaves * 64) void quant_rows_gelu_table(
     const uint16_t* __restrict__ x, int64_t rows, int64_t cols, int64_t ld,
     uint8_t* __restrict__ codes, float* __restrict__ scale_out) {
   __shared__ __attribute__((aligned(16))) uint16_t tab[65536];
-  for (int i = threadIdx.x; i < 65536 / 8; i += kRowTabWaves * 64)
-    ((u32x4_t*)tab)[i] = ((const u32x4_t*)kGeluTable)[i];
+  load_table<kRowTabWaves>(tab);
+  __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   const int nchunk = (int)(cols >> 3);
   const int64_t stride = (int64_t)gridDim.x * kRowTabWaves;
@@ -312,16 +366,6 @@ __global__ __launch_bounds__(kThreads) void quant_rows_generic(
 // ---------------------------------------------------------------------------
 // Tensor mode.
 // ---------------------------------------------------------------------------
-FVSR_DEV float block_max(float m, float* red) {
-  m = wave_max_abs(m);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-  __syncthreads();
-  float r = red[0];
-#pragma unroll
-  for (int w = 1; w < kWaves; ++w) r = fmaxf(r, red[w]);
-  return r;
-}
-
 // Partial |x| maxima: workgroup b covers rows b, b+G, ... (one wave per row).
 // VEC: bf16 rows in 16-byte chunks; otherwise element loads of type dt.
 template <bool GELU, bool VEC>
@@ -334,18 +378,17 @@ __global__ __launch_bounds__(kThreads) void amax_partial(
   for (int64_t row = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6); row < rows;
        row += (int64_t)gridDim.x * kWaves) {
     if (VEC) {
-      const uint16_t* xr = (const uint16_t*)x + row * ld;
-      for (int64_t c = lane; c < (cols >> 3); c += 64) {
-        u32x4_t v = *(const u32x4_t*)(xr + c * 8);
-        if (GELU) v = gelu_chunk(v);
-        m = fmaxf(m, chunk_absmax(v));
-      }
+      // a repeated chunk changes no maximum
+      for_chunks<kChunkLoads>((const uint16_t*)x + row * ld, cols >> 3, lane,
+                              [&](int64_t, const u32x4_t& v) {
+                                m = fmaxf(m, chunk_absmax(GELU ? gelu_chunk(v) : v));
+                              });
     } else {
       for (int64_t c = lane; c < cols; c += 64)
         m = fmaxf(m, fabsf(load_val<GELU>(x, dt, row * ld + c)));
     }
   }
-  m = block_max(m, red);
+  m = block_max<kWaves>(m, red);
   if (threadIdx.x == 0) part[blockIdx.x] = m;
 }
 
@@ -354,20 +397,18 @@ __global__ __launch_bounds__(kThreads) void max_reduce_signed(const float* __res
                                                               int64_t n, float* __restrict__ part) {
   __shared__ float red[kWaves];
   float m = -__builtin_huge_valf();
-  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kThreads)
-    m = fmaxf(m, in[i]);
+  const int64_t stride = (int64_t)gridDim.x * kThreads;
+  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += 4 * stride) {
+    float v[4];  // four loads in flight (past the end the last value again)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = in[clamp_chunk(i + u * stride, n)];
+    m = fmaxf(m, fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])));
+  }
   m = wave_max(m);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
   if (threadIdx.x == 0)
     part[blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-}
-
-FVSR_DEV float reduce_partials(const float* __restrict__ part, int nparts, float* red) {
-  float m = 0.0f;
-  for (int i = threadIdx.x; i < nparts; i += kThreads) m = fmaxf(m, part[i]);
-  return block_max(m, red);
 }
 
 // Codes against the tensor's scale (the partial maxima reduced again by every
@@ -379,7 +420,7 @@ __global__ __launch_bounds__(kThreads) void quant_tensor(
     const float* __restrict__ part, int nparts, uint8_t* __restrict__ codes,
     float* __restrict__ scale_out) {
   __shared__ float red[kWaves];
-  const float amax = reduce_partials(part, nparts, red);
+  const float amax = block_max<kWaves>(max_partials<kThreads>(part, nparts), red);
   const float s = qscale(amax), r = 1.0f / s;
   if (blockIdx.x == 0 && threadIdx.x == 0) scale_out[0] = act_scale(amax);
   const int lane = threadIdx.x & 63;
@@ -387,12 +428,13 @@ __global__ __launch_bounds__(kThreads) void quant_tensor(
        row += (int64_t)gridDim.x * kWaves) {
     uint8_t* qr = codes + row * cols;
     if (VEC) {
-      const uint16_t* xr = (const uint16_t*)x + row * ld;
-      for (int64_t c = lane; c < (cols >> 3); c += 64) {
-        u32x4_t v = *(const u32x4_t*)(xr + c * 8);
-        if (GELU) v = gelu_chunk(v);
-        *(u32x2_t*)(qr + c * 8) = chunk_codes_fma(v, r, qscale_fin(s));
-      }
+      const int64_t n = cols >> 3;
+      for_chunks<kChunkLoads>((const uint16_t*)x + row * ld, n, lane,
+                              [&](int64_t c, const u32x4_t& v) {
+                                if (c < n)
+                                  *(u32x2_t*)(qr + c * 8) = chunk_codes_fma(
+                                      GELU ? gelu_chunk(v) : v, r, qscale_fin(s));
+                              });
     } else {
       for (int64_t c = lane; c < cols; c += 64) {
         float q = clamp448(load_val<GELU>(x, dt, row * ld + c) / s);
@@ -410,9 +452,7 @@ __global__ __launch_bounds__(kThreads) void gelu_amax_from_hmax(
     const uint16_t* __restrict__ h, int64_t rows, int64_t cols, const float* __restrict__ hpart,
     int nh, float* __restrict__ gpart) {
   __shared__ float red[kWaves];
-  float hm = -__builtin_huge_valf();
-  for (int i = threadIdx.x; i < nh; i += kThreads) hm = fmaxf(hm, hpart[i]);
-  hm = wave_max(hm);
+  float hm = wave_max(max_partials<kThreads>(hpart, nh));
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = hm;
   __syncthreads();
   hm = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
@@ -427,7 +467,7 @@ __global__ __launch_bounds__(kThreads) void gelu_amax_from_hmax(
   for (int64_t row = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6); row < rows;
        row += (int64_t)gridDim.x * kWaves)
     for (int64_t c = lane; c < cols; c += 64) m = fmaxf(m, fabsf(gelu_tanh_bf16(bf2f(h[row * cols + c]))));
-  m = block_max(m, red);
+  m = block_max<kWaves>(m, red);
   if (threadIdx.x == 0) gpart[blockIdx.x] = m;
 }
 
@@ -471,7 +511,7 @@ __global__ __launch_bounds__(kThreads) void quant_weight_tensor(
     const void* __restrict__ w, int dt, int64_t n, int64_t k, const float* __restrict__ part,
     int nparts, uint8_t* __restrict__ codes, float* __restrict__ scale_out) {
   __shared__ float red[kWaves];
-  const float s = weight_scale(reduce_partials(part, nparts, red), dt);
+  const float s = weight_scale(block_max<kWaves>(max_partials<kThreads>(part, nparts), red), dt);
   if (blockIdx.x == 0 && threadIdx.x == 0) scale_out[0] = s;
   const int64_t total = n * k;
   for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < total;
@@ -482,9 +522,12 @@ __global__ __launch_bounds__(kThreads) void quant_weight_tensor(
 // ---------------------------------------------------------------------------
 // Host side.
 // ---------------------------------------------------------------------------
+// Workgroups of the tensor-mode passes, one partial maximum each: at most
+// kMaxPartials, every wave the same number of rows but the last ones (8448
+// rows: 704 workgroups of 3 rows a wave, not 1024 of which 64 have a third).
 int partial_blocks(int64_t rows) {
-  int64_t b = (rows + kWaves - 1) / kWaves;
-  return (int)(b < kMaxPartials ? (b > 0 ? b : 1) : kMaxPartials);
+  const int64_t b = (rows + kWaves - 1) / kWaves, per = (b + kMaxPartials - 1) / kMaxPartials;
+  return b > 0 ? (int)((b + per - 1) / per) : 1;
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
@@ -501,6 +544,12 @@ int64_t cu_count() {
   return cus;
 }
 
+// Workgroups of the table kernels: the rows are spread over all CUs before any
+// CU takes a second one (a row's 8960 lookups keep a CU's LDS busy for ~1.1
+// us, so eight rows on one CU in eight would take as long as on all of them;
+// 512 rows 10.1 -> 6.9 us with the table fill above, 1152 10.8 -> 10.1).
+int64_t table_blocks(int64_t rows) { return std::min(rows, cu_count()); }
+
 template <bool GELU>
 int launch_rows(const uint16_t* x, int64_t rows, int64_t cols, int64_t ld, uint8_t* q,
                 float* s, hipStream_t st) {
@@ -508,8 +557,7 @@ int launch_rows(const uint16_t* x, int64_t rows, int64_t cols, int64_t ld, uint8
   const bool vec = (cols % 8 == 0) && (ld % 8 == 0) && aligned16(x) && aligned16(q);
   const int64_t vpl = (cols / 8 + 63) / 64;
   if (GELU && vec && vpl <= 18) {
-    const int64_t want = (rows + kRowTabWaves - 1) / kRowTabWaves;
-    const int64_t g = want < cu_count() ? want : cu_count();
+    const int64_t g = table_blocks(rows);
     hipLaunchKernelGGL((quant_rows_gelu_table<18>), dim3((unsigned)g), dim3(kRowTabWaves * 64), 0,
                        st, x, rows, cols, ld, q, s);
   } else if (vec && vpl <= 3) {
@@ -529,8 +577,7 @@ int launch_rows(const uint16_t* x, int64_t rows, int64_t cols, int64_t ld, uint8
 void launch_gelu_tensor_codes(const uint16_t* x, int64_t rows, int64_t cols, int64_t ld,
                               const float* part, int P, uint8_t* q, float* s, hipStream_t st) {
   if ((cols / 8 + 63) / 64 <= 18) {
-    const int64_t want = (rows + kTabWaves - 1) / kTabWaves;
-    const int64_t g = want < cu_count() ? want : cu_count();
+    const int64_t g = table_blocks(rows);
     hipLaunchKernelGGL((quant_tensor_gelu_table<18>), dim3((unsigned)g), dim3(kTabWaves * 64), 0,
                        st, x, rows, cols, ld, part, P, q, s);
   } else {
@@ -558,9 +605,7 @@ int launch_tensor(const uint16_t* x, int64_t rows, int64_t cols, int64_t ld, uin
   const bool vec = (cols % 8 == 0) && (ld % 8 == 0) && aligned16(x) && aligned16(q);
   if (vec && GELU && (cols / 8 + 63) / 64 <= 18) {
     // both passes by table; the grid is persistent, one partial per workgroup
-    const int64_t want = (rows + kTabWaves - 1) / kTabWaves;
-    int64_t g = want < cu_count() ? want : cu_count();
-    g = g < P ? g : P;
+    const int64_t g = std::min(table_blocks(rows), (int64_t)P);
     hipLaunchKernelGGL((amax_gelu_table<18>), dim3((unsigned)g), dim3(kTabWaves * 64), 0, st, x,
                        rows, cols, ld, ws);
     hipLaunchKernelGGL((quant_tensor_gelu_table<18>), dim3((unsigned)g), dim3(kTabWaves * 64), 0,
