@@ -28,6 +28,11 @@ FVSR_DEV uint32_t bf16_bits(float f) {
 }
 FVSR_DEV float bf16_val(float f) { return __uint_as_float(bf16_bits(f) << 16); }
 
+// Quotient and remainder of block counts and indexes: below 2^31 by the host's
+// checks, so 32-bit (a 64-bit division is a few hundred instructions).
+FVSR_DEV int div32(int64_t a, int64_t b) { return (int)((uint32_t)a / (uint32_t)b); }
+FVSR_DEV int mod32(int64_t a, int64_t b) { return (int)((uint32_t)a % (uint32_t)b); }
+
 FVSR_DEV double wave_sum_f64(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
@@ -52,7 +57,7 @@ __global__ __launch_bounds__(kPoolWaves * 64) void pool_kernel(
   __shared__ double part[kPoolWaves - 1][8][64];
   // The channel slices of one block are neighbours in dispatch order.
   const int64_t ny = (C + 511) / 512;
-  const int64_t blk = blockIdx.x / ny, y = blockIdx.x % ny;
+  const int64_t blk = div32(blockIdx.x, ny), y = mod32(blockIdx.x, ny);
   const bool is_q = blk < NQ;
   const int64_t n = is_q ? blk : blk - NQ;
   const uint16_t* x = is_q ? q : k;
@@ -107,70 +112,83 @@ __global__ __launch_bounds__(kPoolWaves * 64) void pool_kernel(
   }
 }
 
-// Four query blocks l0..l0+3 of one head h per workgroup.  Pass 1: thread m
-// (m = tid, tid+256, ...) forms the four masked scores of key block m, reading
-// each avg_k value once for the four dot products (query values as fp64 in
-// LDS, four 16-byte key loads kept in flight); pass 2: wave w takes row l0+w,
-// its maximum, exponentials and sum by wave reductions, and writes the
-// softmax as bf16 bits to attn[h][l0+w][:] and, for the threshold search, the
-// row's histogram of nonzero patterns by high byte to hist[h][l0+w][0..127]
-// (attn <= 1 or the NaN 0x7fc0, so the high byte is below 128).
+// Four query blocks l0..l0+3 of one head h per workgroup.  Pass 1: the masked
+// scores, in fp64 on v_mfma_f64_4x4x4 (four blocks of 4 x 4 outputs: 4 query
+// blocks x 16 key blocks x 4 channels per instruction; lane l feeds query
+// block l % 4, key block l % 16 and channels of group l / 16, and holds the
+// score of query block l / 16 and key block l % 16).  A wave takes 64 key
+// blocks at a time, each lane 8-channel chunks l / 16 + 4 g of its rows, all
+// loads of 128 channels in flight together.  (Dot products by fp64 fmas with
+// the query values broadcast from LDS read the LDS 256 times per key block:
+// 11.5 us at 12 heads x 66 x 198 blocks against 8.4 here.)  Pass 2: wave w takes row l0+w, its maximum, exponentials and sum by
+// wave reductions, and writes the softmax as bf16 bits to attn[h][l0+w][:]
+// and, for the threshold search, the row's histogram of nonzero patterns by
+// high byte to hist[h][l0+w][0..127] (attn <= 1 or the NaN 0x7fc0, so the high
+// byte is below 128).
 constexpr int kRowsPerScoreWg = 4;
+constexpr int kKeyTiles = 4;  // 16-block key tiles per wave at a time
 
 __global__ __launch_bounds__(kThreads) void score_softmax_kernel(
     const uint16_t* __restrict__ avg_q, const uint16_t* __restrict__ avg_k, int64_t H, int64_t D,
     int64_t NQ, int64_t NK, const uint8_t* __restrict__ local, int64_t sq, int64_t sk,
     float inv_sqrt_d, uint16_t* __restrict__ attn, uint16_t* __restrict__ hist) {
-  extern __shared__ double smem_d[];  // query values [4][D] (fp64), scores [4][NK] (fp32)
+  extern __shared__ float srow[];  // scores [4][NK]
   __shared__ int rh[kRowsPerScoreWg][128];
   constexpr int R = kRowsPerScoreWg;
   const int64_t groups = (NQ + R - 1) / R;
-  const int64_t h = blockIdx.x / groups, l0 = (blockIdx.x % groups) * R;
+  const int64_t h = div32(blockIdx.x, groups), l0 = (int64_t)mod32(blockIdx.x, groups) * R;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t C = H * D;
-  double* aq = smem_d;
-  float* srow = (float*)(smem_d + R * D);
-  for (int64_t i = tid; i < R * D; i += kThreads) {
-    const int64_t l = l0 + i / D;
-    aq[i] = l < NQ ? (double)bf2f(avg_q[l * C + h * D + i % D]) : 0.0;
-  }
+  const int64_t C = H * D, nch = D / 8;
   for (int i = tid; i < R * 128; i += kThreads) rh[i / 128][i % 128] = 0;
-  __syncthreads();
-  const int64_t nch = D / 8;
-  for (int64_t m = tid; m < NK; m += kThreads) {
-    const u32x4_t* ak = (const u32x4_t*)(avg_k + m * C + h * D);
-    double p[R] = {};
-    auto chunk = [&](const u32x4_t& v, int64_t c) {
-      const double* a = aq + 8 * c;
+  const int64_t lq = l0 + (lane & 3) < NQ ? l0 + (lane & 3) : NQ - 1;
+  const u32x4_t* aq = (const u32x4_t*)(avg_q + lq * C + h * D);
+  const u32x4_t zero = {0u, 0u, 0u, 0u};
+  for (int64_t m0 = wave * (16 * kKeyTiles); m0 < NK; m0 += (kThreads / 64) * 16 * kKeyTiles) {
+    const u32x4_t* ak[kKeyTiles];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const double k0 = (double)bf_lo(v[i]), k1 = (double)bf_hi(v[i]);
+    for (int t = 0; t < kKeyTiles; ++t) {
+      const int64_t m = m0 + t * 16 + (lane & 15);
+      ak[t] = (const u32x4_t*)(avg_k + (m < NK ? m : NK - 1) * C + h * D);
+    }
+    double p[kKeyTiles] = {};
+    for (int64_t c0 = 0; c0 < nch; c0 += 16) {
+      u32x4_t a[4], b[kKeyTiles][4];
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          p[r] = __builtin_fma(a[r * D + 2 * i], k0, p[r]);
-          p[r] = __builtin_fma(a[r * D + 2 * i + 1], k1, p[r]);
+      for (int g = 0; g < 4; ++g) {
+        const int64_t c = c0 + 4 * g + (lane >> 4);
+        const bool in = c < nch;  // chunks past the end count as zeros
+        const int64_t cc = in ? c : 0;
+        a[g] = aq[cc];
+        if (!in) a[g] = zero;
+#pragma unroll
+        for (int t = 0; t < kKeyTiles; ++t) {
+          b[t][g] = ak[t][cc];
+          if (!in) b[t][g] = zero;
         }
       }
-    };
-    const u32x4_t zero = {0u, 0u, 0u, 0u};
-    u32x4_t v0 = ak[0], v1 = nch > 1 ? ak[1] : zero, v2 = nch > 2 ? ak[2] : zero,
-            v3 = nch > 3 ? ak[3] : zero;
-#pragma unroll 1
-    for (int64_t c = 0; c < nch; c += 4) {
-      chunk(v0, c);
-      if (c + 4 < nch) v0 = ak[c + 4];
-      if (c + 1 < nch) chunk(v1, c + 1);
-      if (c + 5 < nch) v1 = ak[c + 5];
-      if (c + 2 < nch) chunk(v2, c + 2);
-      if (c + 6 < nch) v2 = ak[c + 6];
-      if (c + 3 < nch) chunk(v3, c + 3);
-      if (c + 7 < nch) v3 = ak[c + 7];
-    }
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const bool allowed = local[((l0 + r) % sq) * sk + m % sk] != 0;
-      srow[r * NK + m] =
-          allowed ? bf16_val(bf16_val((float)p[r]) * inv_sqrt_d) : -__builtin_huge_valf();
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int hf = 0; hf < 2; ++hf) {
+            const double x = (double)(hf ? bf_hi(a[g][i]) : bf_lo(a[g][i]));
+#pragma unroll
+            for (int t = 0; t < kKeyTiles; ++t)
+              p[t] = __builtin_amdgcn_mfma_f64_4x4x4f64(
+                  x, (double)(hf ? bf_hi(b[t][g][i]) : bf_lo(b[t][g][i])), p[t], 0, 0, 0);
+          }
+    }
+    const int64_t r = lane >> 4;
+    const uint8_t* lrow = local + (int64_t)mod32(l0 + r, sq) * sk;
+#pragma unroll
+    for (int t = 0; t < kKeyTiles; ++t) {
+      const int64_t m = m0 + t * 16 + (lane & 15);
+      if (m < NK) {
+        const bool allowed = lrow[mod32(m, sk)] != 0;
+        srow[r * NK + m] =
+            allowed ? bf16_val(bf16_val((float)p[t]) * inv_sqrt_d) : -__builtin_huge_valf();
+      }
     }
   }
   __syncthreads();
@@ -181,6 +199,7 @@ __global__ __launch_bounds__(kThreads) void score_softmax_kernel(
     for (int64_t m = lane; m < NK; m += 64) mx = fmaxf(mx, row[m]);
     mx = wave_max(mx);
     double sum = 0.0;
+#pragma unroll 4
     for (int64_t m = lane; m < NK; m += 64) {
       const float e = (float)exp((double)(row[m] - mx));
       row[m] = e;
@@ -241,35 +260,49 @@ FVSR_DEV int2 find_bin(const int* hist, int r) {
 // 0.  Otherwise the rows' high-byte histograms give the threshold's high byte
 // and its rank r2 among the values sharing it; one pass over the slab then
 // builds the low-byte histogram of those values in LDS.
+// One workgroup per (head, time row) is all there is, so it takes as many
+// threads as it can: with 256 the histogram rows and the slab came in 5 + 4
+// batches of dependent loads at 66 x 198 blocks (8.3 us; 4.6 with 1024).
 constexpr int kSelPer = 16;
+constexpr int kThrThreads = 1024;
 
-__global__ __launch_bounds__(kThreads) void threshold_kernel(const uint16_t* __restrict__ attn,
+__global__ __launch_bounds__(kThrThreads) void threshold_kernel(const uint16_t* __restrict__ attn,
                                                              const uint16_t* __restrict__ hist,
                                                              int64_t NQ, int64_t NK,
                                                              int64_t q_temporal, int64_t topk,
                                                              uint32_t* __restrict__ thr) {
   __shared__ int bins[256];
-  __shared__ int upper[128];
+  __shared__ int upper[kThrThreads];
   __shared__ int2 pick;
-  const int64_t h = blockIdx.x / q_temporal, t = blockIdx.x % q_temporal;
-  const int64_t S = NQ / q_temporal, n = S * NK;
+  const int64_t h = div32(blockIdx.x, q_temporal), t = mod32(blockIdx.x, q_temporal);
+  const int64_t S = div32(NQ, q_temporal), n = S * NK;
   const int tid = threadIdx.x;
   const int r = (int)((topk < n - 1 ? topk : n - 1) + 1);
 
-  // High-byte totals: thread tid sums bin tid % 128 over rows of parity tid / 128.
+  // High-byte totals: thread tid sums bin tid % 128 over rows tid / 128 + 8 i.
+  constexpr int kRowStep = kThrThreads / 128;
   const uint16_t* hs = hist + (h * NQ + t * S) * 128;
   int c = 0;
-  for (int64_t r0 = tid >> 7; r0 < S; r0 += 16) {
+  for (int64_t r0 = tid >> 7; r0 < S; r0 += 8 * kRowStep) {
     uint32_t x[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = r0 + 2 * u < S ? hs[(r0 + 2 * u) * 128 + (tid & 127)] : 0u;
+    for (int u = 0; u < 8; ++u) {
+      const int64_t rr = r0 + u * kRowStep;
+      x[u] = rr < S ? hs[rr * 128 + (tid & 127)] : 0u;
+    }
 #pragma unroll
     for (int u = 0; u < 8; ++u) c += (int)x[u];
   }
-  if (tid >= 128) upper[tid - 128] = c;
+  upper[tid] = c;
   __syncthreads();
-  if (tid < 128) bins[tid] = c + upper[tid];
-  else bins[tid] = 0;
+  if (tid < 256) {
+    int total = 0;
+    if (tid < 128) {
+#pragma unroll
+      for (int u = 0; u < kRowStep; ++u) total += upper[u * 128 + tid];
+    }
+    bins[tid] = total;
+  }
   __syncthreads();
   if (tid < 64) {
     const int2 f = find_bin(bins, r);
@@ -281,14 +314,14 @@ __global__ __launch_bounds__(kThreads) void threshold_kernel(const uint16_t* __r
     if (tid == 0) thr[blockIdx.x] = 0u;
     return;
   }
-  bins[tid] = 0;
+  if (tid < 256) bins[tid] = 0;
   __syncthreads();
   const uint16_t* vals = attn + (h * NQ + t * S) * NK;
-  for (int64_t base = 0; base < n; base += kSelPer * kThreads) {
+  for (int64_t base = 0; base < n; base += kSelPer * kThrThreads) {
     uint32_t v[kSelPer];
 #pragma unroll
     for (int i = 0; i < kSelPer; ++i) {
-      const int64_t idx = base + i * kThreads + tid;
+      const int64_t idx = base + i * kThrThreads + tid;
       v[i] = idx < n ? (uint32_t)vals[idx] : 0u;
     }
 #pragma unroll
@@ -314,8 +347,8 @@ __global__ __launch_bounds__(kThreads) void index_kernel(const uint16_t* __restr
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
   if (row >= rows) return;
-  const int64_t h = row / NQ, l = row % NQ, S = NQ / q_temporal;
-  const float th = bf2f((uint16_t)thr[h * q_temporal + l / S]);
+  const int64_t h = div32(row, NQ), l = mod32(row, NQ), S = div32(NQ, q_temporal);
+  const float th = bf2f((uint16_t)thr[h * q_temporal + div32(l, S)]);
   const uint16_t* ar = attn + row * NK;
   int base = 0;
   for (int64_t c0 = 0; c0 < NK; c0 += 8 * 64) {
@@ -371,7 +404,7 @@ extern "C" int fvsr_draft_block_mask(const void* q, int64_t q_tok_stride, const 
       ((uintptr_t)workspace & 15))
     return FVSR_EUNSUPPORTED;
   if (workspace_floats < fvsr_draft_workspace_floats(H, D, NQ, NK)) return FVSR_EWORKSPACE;
-  // LDS holds 4 * D doubles and 4 * NK floats (at most 62 KB).
+  // LDS holds 4 * NK floats; 2 * D + NK keeps the bound of an earlier layout.
   if (2 * D + NK > 3968 || (NQ / q_temporal) * NK > 0x7fffffff || H * NQ > 0x7fffffff ||
       (NQ + NK) * ((H * D + 511) / 512) > 0x7fffffff)
     return FVSR_EUNSUPPORTED;
@@ -387,9 +420,9 @@ extern "C" int fvsr_draft_block_mask(const void* q, int64_t q_tok_stride, const 
   uint32_t* thr = (uint32_t*)(hist + align64(H * NQ * 128));
   const int64_t groups = (NQ + kRowsPerScoreWg - 1) / kRowsPerScoreWg;
   hipLaunchKernelGGL(score_softmax_kernel, dim3((unsigned)(H * groups)), dim3(kThreads),
-                     kRowsPerScoreWg * (D * sizeof(double) + NK * sizeof(float)), st, avg,
+                     kRowsPerScoreWg * NK * sizeof(float), st, avg,
                      avg + NQ * C, H, D, NQ, NK, local, sq, sk, inv_sqrt_d, attn, hist);
-  hipLaunchKernelGGL(threshold_kernel, dim3((unsigned)(H * q_temporal)), dim3(kThreads), 0, st,
+  hipLaunchKernelGGL(threshold_kernel, dim3((unsigned)(H * q_temporal)), dim3(kThrThreads), 0, st,
                      attn, hist, NQ, NK, q_temporal, topk, thr);
   const int64_t rows = H * NQ;
   hipLaunchKernelGGL(index_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(kThreads), 0, st, attn,

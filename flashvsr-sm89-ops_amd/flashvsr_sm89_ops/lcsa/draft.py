@@ -9,7 +9,7 @@ joint top-k per (head, query time row); ``keep = attn > thr``.
 For bf16 q/k every stage is rounded to bf16 as torch rounds bf16 tensors
 (mean, einsum, division by sqrt(D), softmax), so ties at the threshold fall
 as they do in the reference.  ``fvsr_draft_block_mask`` runs the whole chain
-in three launches and can write the block index (sel, cnt) that the
+in four launches and can write the block index (sel, cnt) that the
 attention kernel consumes directly, without the bool mask or a host sync.
 """
 from __future__ import annotations
@@ -71,7 +71,8 @@ def draft_index(q: torch.Tensor, k: torch.Tensor, *, nheads: int, q_temporal: in
         raise ValueError(f"NQ={NQ}, NK={NK} must tile q_temporal={q_temporal} and the "
                          f"local mask {sq}x{sk}")
     dev = q.device
-    keep = torch.empty((nheads, NQ, NK), dtype=torch.uint8, device=dev) if want_keep else None
+    # bool: the kernel writes bytes 0 and 1
+    keep = torch.empty((nheads, NQ, NK), dtype=torch.bool, device=dev) if want_keep else None
     sel = cnt = None
     if want_index:
         sel = torch.empty((nheads, NQ, max(NK, 1)), dtype=torch.int32, device=dev)
@@ -86,8 +87,8 @@ def draft_index(q: torch.Tensor, k: torch.Tensor, *, nheads: int, q_temporal: in
     _lib.check(rc, "draft_block_mask")
     index = (sel, cnt, max(NK, 1)) if want_index else None
     if want_keep and want_index:
-        return index, keep.bool()
-    return keep.bool() if want_keep else index
+        return index, keep
+    return keep if want_keep else index
 
 
 def draft_block_mask(q_w: torch.Tensor, k_w: torch.Tensor, nheads: int, q_temporal: int,
