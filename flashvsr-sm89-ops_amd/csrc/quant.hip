@@ -522,8 +522,14 @@ __global__ __launch_bounds__(kThreads) void quant_weight_tensor(
 // ---------------------------------------------------------------------------
 // Host side.
 // ---------------------------------------------------------------------------
-// Workgroups of the tensor-mode passes, one partial maximum each: at most
-// kMaxPartials, every wave the same number of rows but the last ones (8448
+// Partial maxima a caller's workspace holds in tensor mode.
+int partial_floats(int64_t rows) {
+  const int64_t b = (rows + kWaves - 1) / kWaves;
+  return (int)(b < kMaxPartials ? (b > 0 ? b : 1) : kMaxPartials);
+}
+
+// Workgroups of the tensor-mode passes, one partial maximum each (at most
+// partial_floats): every wave the same number of rows but the last ones (8448
 // rows: 704 workgroups of 3 rows a wave, not 1024 of which 64 have a third).
 int partial_blocks(int64_t rows) {
   const int64_t b = (rows + kWaves - 1) / kWaves, per = (b + kMaxPartials - 1) / kMaxPartials;
@@ -629,7 +635,7 @@ int launch_tensor(const uint16_t* x, int64_t rows, int64_t cols, int64_t ld, uin
 
 extern "C" int64_t fvsr_quant_workspace_floats(int64_t rows, int64_t cols, int mode) {
   (void)cols;
-  return mode == FVSR_SCALE_ROW ? 0 : partial_blocks(rows);
+  return mode == FVSR_SCALE_ROW ? 0 : partial_floats(rows);
 }
 
 extern "C" int fvsr_quant_fp8(const void* x, int64_t rows, int64_t cols, int64_t ld, int mode,
@@ -645,7 +651,7 @@ extern "C" int fvsr_quant_fp8(const void* x, int64_t rows, int64_t cols, int64_t
   if (mode == FVSR_SCALE_ROW)
     return gelu ? launch_rows<true>(xp, rows, cols, ld, qp, scale_out, st)
                 : launch_rows<false>(xp, rows, cols, ld, qp, scale_out, st);
-  if (!workspace || workspace_floats < partial_blocks(rows)) return FVSR_EWORKSPACE;
+  if (!workspace || workspace_floats < partial_floats(rows)) return FVSR_EWORKSPACE;
   return gelu ? launch_tensor<true>(xp, rows, cols, ld, qp, scale_out, workspace, st)
               : launch_tensor<false>(xp, rows, cols, ld, qp, scale_out, workspace, st);
 }
@@ -658,7 +664,7 @@ extern "C" int fvsr_gelu_quant_fp8_tensor(const void* h, int64_t rows, int64_t c
   if (rows == 0 || cols == 0) return FVSR_OK;
   if (!h || !codes || !scale_out || !hmax_part) return FVSR_EINVAL;
   const int P = partial_blocks(rows);
-  if (!workspace || workspace_floats < 2 * P) return FVSR_EWORKSPACE;
+  if (!workspace || workspace_floats < 2 * partial_floats(rows)) return FVSR_EWORKSPACE;
   hipStream_t st = (hipStream_t)stream;
   const uint16_t* hp = (const uint16_t*)h;
   uint8_t* qp = (uint8_t*)codes;
@@ -694,7 +700,7 @@ extern "C" int fvsr_quant_weight_fp8_dt(const void* w, int w_dtype, int64_t n, i
     return fvsr_launch_status();
   }
   const int P = partial_blocks(n);
-  if (!workspace || workspace_floats < P) return FVSR_EWORKSPACE;
+  if (!workspace || workspace_floats < partial_floats(n)) return FVSR_EWORKSPACE;
   hipLaunchKernelGGL((amax_partial<false, false>), dim3(P), dim3(kThreads), 0, st, w, w_dtype, n,
                      k, k, workspace);
   hipLaunchKernelGGL(quant_weight_tensor, dim3(P), dim3(kThreads), 0, st, w, w_dtype, n, k,
@@ -732,7 +738,7 @@ extern "C" int fvsr_quant_fp8_dt(const void* x, int x_dtype, int64_t rows, int64
                          ld, qp, scale_out);
     return fvsr_launch_status();
   }
-  if (!workspace || workspace_floats < partial_blocks(rows)) return FVSR_EWORKSPACE;
+  if (!workspace || workspace_floats < partial_floats(rows)) return FVSR_EWORKSPACE;
   return gelu ? launch_tensor_scalar<true>(x, x_dtype, rows, cols, ld, qp, scale_out, workspace, st)
               : launch_tensor_scalar<false>(x, x_dtype, rows, cols, ld, qp, scale_out, workspace,
                                             st);
@@ -792,7 +798,7 @@ extern "C" int fvsr_quant_fp8_noalloc(const void* x, int64_t rows, int64_t cols,
   if (mode == FVSR_SCALE_ROW)
     return gelu ? launch_rows<true>(xp, rows, cols, ld, qp, scale_out, st)
                 : launch_rows<false>(xp, rows, cols, ld, qp, scale_out, st);
-  if (partial_blocks(rows) > kScratchFloats) return FVSR_EWORKSPACE;
+  if (partial_floats(rows) > kScratchFloats) return FVSR_EWORKSPACE;
   int dev = 0;
   if ((st ? hipStreamGetDevice(st, &dev) : hipGetDevice(&dev)) != hipSuccess) return FVSR_EHIP;
   float* ws = nullptr;
