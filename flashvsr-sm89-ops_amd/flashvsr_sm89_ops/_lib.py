@@ -107,6 +107,31 @@ def lib():
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The extension with the native host side of quantisation and GEMM
+    (csrc/host_ops.cpp), bound to the loaded library's functions; like the
+    library it must be built."""
+    global _host
+    if _host is None:
+        L = lib()
+        with _lock:
+            if _host is None:
+                try:
+                    from . import _fvsr_host as h
+                except ImportError as e:
+                    raise RuntimeError(
+                        "flashvsr_sm89_ops: _fvsr_host.so is not built. Build it with "
+                        "`python flashvsr-sm89-ops_amd/build.py`.") from e
+                h.bind(*(ctypes.cast(getattr(L, n), _P).value for n in (
+                    "fvsr_quant_workspace_floats", "fvsr_quant_fp8_dt", "fvsr_fp8_gemm",
+                    "fvsr_gemm_amax_parts")))
+                _host = h
+    return _host
+
+
 def check(rc: int, what: str):
     if rc != FVSR_OK:
         raise RuntimeError(f"{what} failed: {_ERR.get(rc, rc)} (status {rc})")

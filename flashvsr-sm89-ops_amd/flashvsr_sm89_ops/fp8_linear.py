@@ -89,6 +89,11 @@ def fp8_gemm(x8: torch.Tensor, s: torch.Tensor, w8: torch.Tensor, w_scale: torch
     (same row stride) and ``gate`` [N] bf16.  Every size is checked here,
     before the launch, as torch._scaled_mm checks its operands (reference
     fp8_linear.py:28-30); a mismatch raises ValueError / TypeError."""
+    if x8.is_cuda and out is None and res is None and gate is None and \
+            epilogue == (_lib.EPI_BIAS if amax_part is None else _lib.EPI_ROWMAX):
+        y = _lib.host().gemm(x8, s, w8, w_scale, bias, amax_part)  # plain operands, one native call
+        if y is not None:
+            return y
     _check_gemm_args(x8, s, w8, w_scale, bias, out, epilogue, amax_part, res, gate)
     _lib.require_gpu(x8, s, w8, w_scale, bias, out, amax_part, res, gate)
     M, K = x8.shape

@@ -34,6 +34,10 @@ def quantize_fp8(x2: torch.Tensor, per_token: bool = False):
 def quantize_rows_fp8(x2: torch.Tensor, per_token: bool, gelu: bool, what: str):
     """Activation quantisation of x2 (or of tanh-GELU(x2) rounded to bf16) through
     fvsr_quant_fp8_dt."""
+    if x2.is_cuda:
+        r = _lib.host().quantize(x2, per_token, gelu)  # plain inputs, in one native call
+        if r is not None:
+            return r
     _lib.require_gpu(x2)
     dt = _lib.dtype_code(x2, "x2")
     if x2.dim() != 2:

@@ -1,0 +1,131 @@
+"""The native host side of quantisation and GEMM: the same results as the
+general Python path, which every other call form still reaches."""
+import pytest
+import torch
+
+DEV = "cuda"
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture()
+def general(monkeypatch):
+    """Calls f with the native calls off."""
+    from flashvsr_sm89_ops import _lib
+
+    class Off:
+        quantize = gemm = staticmethod(lambda *a: None)
+
+    def run(f):
+        with monkeypatch.context() as m:
+            m.setattr(_lib, "_host", Off)
+            return f()
+    return run
+
+
+def _same(a, b):
+    if isinstance(a, tuple):
+        assert len(a) == len(b)
+        for x, y in zip(a, b):
+            _same(x, y)
+        return
+    assert a.shape == b.shape and a.dtype == b.dtype and a.stride() == b.stride()
+    assert a.device == b.device and a.requires_grad == b.requires_grad
+    v = torch.uint8 if a.element_size() == 1 else torch.int16 if a.element_size() == 2 else torch.int32
+    assert torch.equal(a.view(v), b.view(v))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("form", ["plain", "rows", "columns", "empty", "param", "transposed"])
+def test_quantize_forms(general, dtype, form):
+    from flashvsr_sm89_ops import _lib
+    from flashvsr_sm89_ops.fp8_ffn import fused_gelu_quant_fp8
+    from flashvsr_sm89_ops.fp8_quant import quantize_fp8
+    x = torch.randn(37, 96, device=DEV).to(dtype)
+    x = {"plain": x, "rows": x[:, :40], "columns": x[:, 8:48], "empty": x[:0],
+         "param": torch.nn.Parameter(x, requires_grad=False), "transposed": x.t()}[form]
+    native = _lib.host().quantize(x, True, False) is not None
+    assert native == (form not in ("empty", "transposed"))
+    for f in (quantize_fp8, fused_gelu_quant_fp8):
+        for per_token in (False, True):
+            _same(f(x, per_token=per_token), general(lambda: f(x, per_token=per_token)))
+
+
+def test_gemm_forms(general):
+    import flashvsr_sm89_ops as fv
+    from flashvsr_sm89_ops import _lib
+    M, N, K = 70, 96, 256
+    x8, s = fv.quantize_fp8(torch.randn(M, K, device=DEV).bfloat16(), per_token=True)
+    w8, ws = fv.quantize_weight_fp8(torch.randn(N, K, device=DEV).bfloat16(), per_channel=True)
+    b = torch.randn(N, device=DEV).bfloat16()
+    one, one0 = s[:1].reshape(1), ws[0]
+    hmax = torch.empty(M, 1, device=DEV)
+    wide = torch.zeros(M, 2 * K, device=DEV).to(torch.float8_e4m3fn)
+    wide[:, :K] = x8
+    forms = [((x8, s, w8, ws, b), {}, True), ((x8, s, w8, ws, None), {}, True),
+             ((x8, one, w8, one0, b), {}, True), ((x8[:1], s[:1], w8, ws, b), {}, True),
+             ((wide[:, :K], s, w8, ws, b), {}, True), ((x8[:0], s[:0], w8, ws, b), {}, None),
+             ((x8, s, w8, ws, b.float()), {}, False), ((x8, s.double(), w8, ws, b), {}, False),
+             ((x8, s, w8, ws, b), dict(epilogue=_lib.EPI_ROWMAX, amax_part=hmax), True),
+             ((x8, s, torch.nn.Parameter(w8, requires_grad=False), ws, b), {}, True)]
+    for args, kw, native in forms:
+        if native is not None:
+            got = _lib.host().gemm(*args, kw.get("amax_part"))
+            assert (got is not None) == native
+        a = fv.fp8_gemm(*args, **kw)
+        part = hmax.clone()
+        _same(a, general(lambda: fv.fp8_gemm(*args, **kw)))
+        assert torch.equal(part, hmax)
+
+
+def test_refusals_and_modes(general):
+    """What the general path refuses stays refused with its own error; calls
+    under a torch mode go through the general path."""
+    import flashvsr_sm89_ops as fv
+    from flashvsr_sm89_ops import _lib
+    x8, s = fv.quantize_fp8(torch.randn(64, 256, device=DEV).bfloat16(), per_token=True)
+    w8, ws = fv.quantize_weight_fp8(torch.randn(96, 256, device=DEV).bfloat16(), per_channel=True)
+    bad = [(x8[:, :128], s, w8, ws), (x8, s[:7], w8, ws), (x8, s, w8, ws[:5]),
+           (x8.view(torch.uint8), s, w8, ws), (x8, s, w8, ws, s.reshape(-1)[:64]),
+           (x8, s.cpu(), w8, ws), (x8[:, 8:], s, w8[:, 8:], ws)]  # the last: unaligned rows
+    for args in bad:
+        kinds = []
+        for call in (lambda: fv.fp8_gemm(*args), lambda: general(lambda: fv.fp8_gemm(*args))):
+            with pytest.raises((ValueError, TypeError, RuntimeError)) as e:
+                call()
+            kinds.append((e.type, str(e.value)))
+        assert kinds[0] == kinds[1]
+    with pytest.raises(TypeError):
+        fv.quantize_fp8(torch.zeros(4, 8, device=DEV, dtype=torch.int32))
+    with pytest.raises(ValueError):
+        fv.quantize_fp8(torch.zeros(4, 8, 2, device=DEV, dtype=torch.bfloat16))
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Seen(TorchDispatchMode):
+        n = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.n += 1
+            return func(*args, **(kwargs or {}))
+
+    x = torch.randn(8, 64, device=DEV).bfloat16()
+    want = fv.quantize_fp8(x, per_token=True)
+    with Seen() as m:
+        assert _lib.host().quantize(x, True, False) is None
+        got = fv.quantize_fp8(x, per_token=True)
+    assert m.n > 0
+    _same(got, want)
+
+
+def test_streams(general):
+    """The launch and the allocations follow torch's current stream."""
+    import flashvsr_sm89_ops as fv
+    side = torch.cuda.Stream()
+    x = torch.randn(2048, 1536, device=DEV).bfloat16()
+    want = fv.quantize_fp8(x)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        with torch.cuda.stream(side):
+            y = (x * 1.0).contiguous()      # on the side stream
+            got = fv.quantize_fp8(y)
+        side.synchronize()
+        _same(got, want)
