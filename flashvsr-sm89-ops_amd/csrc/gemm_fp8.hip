@@ -593,10 +593,21 @@ FVSR_DEV void fast_params(FastParams& fp, const uint8_t LDS_AS* prm, int ip, int
     }
 }
 
-// Convert pass (ip, j) and write it to the staging area.
-template <int MJ>
+// max(m, a, b) in one instruction, a NaN passed over as fmaxf does.
+FVSR_DEV float max3(float m, float a, float b) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(m), "v"(a), "v"(b));
+  return r;
+}
+
+// Convert pass (ip, j) and write it to the staging area.  ROWMAX: vm follows
+// the largest value of the lane's row (before its rounding to bf16, which is
+// monotone): half an instruction per value here, where taking it from the
+// stored bf16 chunks unpacked and compared each (+27 us on 108 at 8448 x 8960
+// x 1536; now +1, and +4 on 206 at 16896).
+template <int EPI, int MJ>
 FVSR_DEV void fast_stage(const v16f (&acc)[4][MJ], const FastParams& fp, float sam,
-                         uint16_t LDS_AS* stg, int ip, int j, int row, int h) {
+                         uint16_t LDS_AS* stg, int ip, int j, int row, int h, float& vm) {
 #pragma unroll
   for (int ii = 0; ii < 2; ++ii)
 #pragma unroll
@@ -605,6 +616,7 @@ FVSR_DEV void fast_stage(const v16f (&acc)[4][MJ], const FastParams& fp, float s
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         y[r] = acc[2 * ip + ii][j][g * 4 + r] * (sam * fp.sb[ii][g][r]) + fp.bias[ii][g][r];
+      if (EPI == FVSR_EPI_ROWMAX) vm = max3(max3(vm, y[0], y[1]), y[2], y[3]);
       *(u32x2_t LDS_AS*)((uint8_t LDS_AS*)stg + epi_off(row, ii * 8 + g * 2 + h)) =
           u32x2_t{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
     }
@@ -630,15 +642,10 @@ FVSR_DEV void fast_read(const uint16_t LDS_AS* stg, u32x4_t (&v)[4], int lane) {
 // allocating those lines in L2 evicted the operand panels the next tiles read
 // (qkv 111 -> 107 us, ffn0 217 -> 207 us, C1 15.5 -> 14.1 us; bit-identical).
 constexpr int kStoreNT = 2;  // aux bits of the raw buffer store: nt
-template <int EPI>
-FVSR_DEV void fast_store(const u32x4_t (&v)[4], float (&vmax)[4], i32x4_t rc, uint32_t voff,
-                         int64_t ldc, int ip, int j) {
+FVSR_DEV void fast_store(const u32x4_t (&v)[4], i32x4_t rc, uint32_t voff, int64_t ldc, int ip,
+                         int j) {
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
-    if (EPI == FVSR_EPI_ROWMAX) {
-#pragma unroll
-      for (int w = 0; w < 4; ++w) vmax[s] = fmaxf(vmax[s], fmaxf(bf_lo(v[s][w]), bf_hi(v[s][w])));
-    }
     const uint32_t off = voff + (uint32_t)((j * 32 + s * 8) * ldc * 2 + ip * 128);
     fvsr_buffer_store_b128(v[s], rc, __builtin_bit_cast(int, off), 0, kStoreNT);
   }
@@ -657,14 +664,12 @@ FVSR_DEV void epi_fast(const v16f (&acc)[4][MJ], uint16_t LDS_AS* stg, const uin
   // block, row group and column half (all in the offset the range check
   // covers).
   const uint32_t voff = (uint32_t)(((mw + (lane >> 3)) * e.ldc + nw + (lane & 7) * 8) * 2);
-  float vmax[MJ][4];
+  float vm[MJ];
 #pragma unroll
-  for (int j = 0; j < MJ; ++j)
-#pragma unroll
-    for (int s = 0; s < 4; ++s) vmax[j][s] = -__builtin_huge_valf();
+  for (int j = 0; j < MJ; ++j) vm[j] = -__builtin_huge_valf();
   FastParams fp;
   fast_params(fp, prm, 0, h);
-  fast_stage<MJ>(acc, fp, sam[0], stg, 0, 0, row, h);
+  fast_stage<EPI, MJ>(acc, fp, sam[0], stg, 0, 0, row, h, vm[0]);
   // Passes p = ip * MJ + j.
 #pragma unroll
   for (int p = 0; p < 2 * MJ; ++p) {
@@ -673,21 +678,20 @@ FVSR_DEV void epi_fast(const v16f (&acc)[4][MJ], uint16_t LDS_AS* stg, const uin
     fast_read(stg, v, lane);
     if (p == MJ - 1) fast_params(fp, prm, 1, h);
     if (p + 1 < 2 * MJ)
-      fast_stage<MJ>(acc, fp, sam[(p + 1) % MJ], stg, (p + 1) / MJ, (p + 1) % MJ, row, h);
-    fast_store<EPI>(v, vmax[j], rc, voff, e.ldc, ip, j);
+      fast_stage<EPI, MJ>(acc, fp, sam[(p + 1) % MJ], stg, (p + 1) / MJ, (p + 1) % MJ, row, h,
+                          vm[(p + 1) % MJ]);
+    fast_store(v, rc, voff, e.ldc, ip, j);
   }
   if (EPI == FVSR_EPI_ROWMAX) {
-    // 8 lanes per row cover 64 columns per pass; both halves = the slab.
+    // The row's other values of the slab are in lane ^ 32.
 #pragma unroll
-    for (int j = 0; j < MJ; ++j)
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        float v = vmax[j][s];
-#pragma unroll
-        for (int o = 4; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-        const int64_t m = mw + j * 32 + s * 8 + (lane >> 3);
-        if ((lane & 7) == 0 && m < M) e.amax_part[m * e.nparts + nw / 128] = v;
-      }
+    for (int j = 0; j < MJ; ++j) {
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(vm[j]),
+                                                       __float_as_uint(vm[j]), false, false);
+      const float v = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+      const int64_t m = mw + j * 32 + row;
+      if (h == 0 && m < M) e.amax_part[m * e.nparts + nw / 128] = round_bf16(v);
+    }
   }
 }
 

@@ -74,3 +74,24 @@ def test_fp8_gemm_rows_do_not_depend_on_the_tile(K):
     full = ops.fp8_gemm(ad, sad, bd, sbd, bi)
     for M in (64, 700, 1152, 2079, 4000, 6200):
         assert torch.equal(ops.fp8_gemm(ad[:M], sad[:M], bd, sbd, bi), full[:M])
+
+
+@pytest.mark.parametrize("M", [300, 2079, 8200])
+def test_rowmax_passes_nans_over(M):
+    """Row maxima of the row-max epilogue ignore NaN outputs (a NaN bias
+    column, a row whose every value is NaN: -inf) and keep infinities."""
+    import flashvsr_sm89_ops as ops
+    from flashvsr_sm89_ops import _lib
+    N, K = 1536, 512
+    a, b, sa, sb, bias = _gemm_inputs(M, N, K, seed=M)
+    sa[3] = np.nan
+    bias = O.from_bf16_bits(bias)
+    bias[5], bias[200], bias[1535] = np.nan, np.inf, -np.inf
+    hmax = torch.empty((M, N // 128), dtype=torch.float32, device=DEV)
+    y = ops.fp8_gemm(codes_dev(a), torch.from_numpy(sa).to(DEV), codes_dev(b),
+                     torch.from_numpy(sb).to(DEV), dev_bf16(O.bf16_bits(bias)),
+                     epilogue=_lib.EPI_ROWMAX, amax_part=hmax)
+    h = host_f(y).reshape(M, N // 128, 128)
+    want = np.where(np.isnan(h), -np.inf, h).max(2)
+    assert np.array_equal(host_f(hmax), want)
+    assert (host_f(hmax)[3] == -np.inf).all() and (np.delete(host_f(hmax), 3, 0)[:, 1] == np.inf).all()
