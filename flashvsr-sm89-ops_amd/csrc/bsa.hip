@@ -305,14 +305,16 @@ FVSR_DEV int64_t query_token(int qb, int qpos, const int32_t* q_map, const WinGe
 
 // QM / KM: how query and key/value block positions become stored token rows
 // (kDirect, kMap or kWin, see above); the output rows are the query rows.
-// DENSE: every key block 0..maxk-1 is kept for every query block (the
+// kDense: every key block 0..maxk-1 is kept for every query block (the
 // cross-attention over the cached prompt, integrate.py:132-143): no block
-// index is read and a workgroup of 8 waves takes two query blocks (waves 0-3
-// and 4-7) over one K/V stream, so the per-unit start-up and the K/V stream
-// are paid once per two query blocks (2 waves per SIMD, as two 4-wave
-// workgroups would give).
-template <int QM, int KM, bool DENSE>
-__global__ __attribute__((amdgpu_flat_work_group_size(DENSE ? 512 : 256, DENSE ? 512 : 256),
+// index is read.  kDensePair: the same with a workgroup of 8 waves taking two
+// query blocks (waves 0-3 and 4-7) over one K/V stream, so the per-unit
+// start-up and the K/V stream are paid once per two query blocks (2 waves per
+// SIMD, as two 4-wave workgroups would give).
+enum { kSparse = 0, kDense = 1, kDensePair = 2 };
+template <int QM, int KM, int MODE>
+__global__ __attribute__((amdgpu_flat_work_group_size(MODE == kDensePair ? 512 : 256,
+                                                      MODE == kDensePair ? 512 : 256),
                           amdgpu_waves_per_eu(2, 2)))
 void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
                     const uint16_t* __restrict__ v, uint16_t* __restrict__ o, int64_t q_ts,
@@ -323,6 +325,7 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
                     int pieces, float* __restrict__ part) {
   __shared__ __attribute__((aligned(1024))) uint8_t stage0[kStage];
   __shared__ __attribute__((aligned(1024))) uint8_t stage1[kStage];
+  constexpr bool DENSE = MODE != kSparse, PAIR = MODE == kDensePair;
   uint8_t LDS_AS* st0 = (uint8_t LDS_AS*)stage0;
   uint8_t LDS_AS* st1 = (uint8_t LDS_AS*)stage1;
   // Workgroup ids are dispatched round robin over the 8 XCDs; give each XCD a
@@ -336,14 +339,14 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
   const int xcd = (blockIdx.x - first) % 8, loc = (blockIdx.x - first) / 8;
   const int slot = xcd < rem ? xcd * (per + 1) + loc : rem * (per + 1) + (xcd - rem) * per + loc;
   const int unit = is_piece ? whole + slot / pieces : slot;
-  constexpr int NW = DENSE ? 8 : 4;
-  const int units_per_head = DENSE ? (NQ + 1) / 2 : NQ;
+  constexpr int NW = PAIR ? 8 : 4;
+  const int units_per_head = PAIR ? (NQ + 1) / 2 : NQ;
   const int h = unit / units_per_head, up = unit % units_per_head;
   const int lane = threadIdx.x & 63, half = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // A dense pair's second query block may lie past NQ (odd NQ): its waves
+  // A pair's second query block may lie past NQ (odd NQ): its waves
   // follow the stream on the last block and store nothing.
-  const int qb_raw = DENSE ? 2 * up + (wave >> 2) : up;
+  const int qb_raw = PAIR ? 2 * up + (wave >> 2) : up;
   const bool q_live = qb_raw < NQ;
   const int qb = q_live ? qb_raw : NQ - 1;
   int n = DENSE ? (int)maxk : cnt[(int64_t)h * NQ + qb];
@@ -441,7 +444,7 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
     return;
   }
   const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-  if (DENSE) {
+  if (PAIR) {
     __syncthreads();  // waves 4-7 stage through stage1, which the last step reads
     if (!q_live) return;
   }
@@ -584,6 +587,16 @@ extern "C" int fvsr_block_index(const uint8_t* keep, int64_t H, int64_t NQ, int6
 
 namespace {
 
+// Compute units of the current device, a multiple of the 8 XCDs.
+int64_t cu_count() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      cus < 8)
+    cus = 256;
+  return cus & ~7;
+}
+
 // How a call's units are laid out: the first `whole` run as one workgroup
 // each, every later one as `pieces` workgroups over parts of its kept blocks
 // (partial results in the caller's workspace, then bsa_combine_kernel).
@@ -607,35 +620,26 @@ struct Split {
 };
 
 Split plan_split(int64_t H, int64_t NQ, int64_t maxk) {
-  const int64_t units = H * NQ;
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      cus < 8)
-    cus = 256;
-  cus &= ~7;
+  const int64_t units = H * NQ, cus = cu_count();
   const Split plain{units, 0, 1};
   const int64_t rest = units % cus;
-#ifdef FVSR_TUNE
-  if (g_split == 1) return plain;
-  if (g_split > 1) return Split{units - rest, rest, g_split};
-#endif
   if (rest == 0 || units >= 6 * cus || (units > cus && 4 * rest > 3 * cus)) return plain;
   const int64_t pieces = std::min({2 * cus / rest, maxk / 4, (int64_t)8});
   return pieces > 1 ? Split{units - rest, rest, (int)pieces} : plain;
 }
 
-template <int QM, int KM, bool DENSE = false>
+template <int QM, int KM, int MODE = kSparse>
 void launch_bsa(const void* q, const void* k, const void* v, void* o, int64_t q_ts, int64_t q_hs,
                 int64_t kv_ts, int64_t kv_hs, int64_t o_ts, int64_t o_hs, const int32_t* sel,
                 const int32_t* cnt, int64_t maxk, int64_t H, int64_t NQ, float scale_log2,
                 const int32_t* q_map, const int32_t* kv_map, WinGeo geo, hipStream_t st,
                 const Split* split = nullptr, float* part = nullptr) {
-  const int64_t units = H * (DENSE ? (NQ + 1) / 2 : NQ);
+  constexpr bool PAIR = MODE == kDensePair;
+  const int64_t units = H * (PAIR ? (NQ + 1) / 2 : NQ);
   const Split sp = split && part ? *split : Split{units, 0, 1};
-  hipLaunchKernelGGL((bsa_fwd_kernel<QM, KM, DENSE>),
+  hipLaunchKernelGGL((bsa_fwd_kernel<QM, KM, MODE>),
                      dim3((unsigned)(sp.whole + sp.rest * sp.pieces)),
-                     dim3(DENSE ? 2 * kThreads : kThreads), 0, st,
+                     dim3(PAIR ? 2 * kThreads : kThreads), 0, st,
                      (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o,
                      q_ts, q_hs, kv_ts, kv_hs, o_ts, o_hs, sel, cnt, maxk, (int)NQ, scale_log2,
                      q_map, kv_map, geo, (int)(aligned16(o) && (o_ts | o_hs) % 8 == 0),
@@ -790,9 +794,19 @@ extern "C" int fvsr_attn_dense(const void* q, const void* k, const void* v, void
   if (rc != FVSR_OK) return rc;
   if (NK > 0x3fffffff) return FVSR_EUNSUPPORTED;
   const WinGeo geo{0, 0, 1, 1};
-  launch_bsa<kDirect, kDirect, true>(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride,
-                                     kv_head_stride, o_tok_stride, o_head_stride, nullptr,
-                                     nullptr, NK, H, NQ, sm_scale * 1.4426950408889634f,
-                                     nullptr, nullptr, geo, (hipStream_t)stream);
+  // Two query blocks per workgroup (one round per CU at a time, start-up and
+  // K/V paid once for both), unless each block finds a CU of its own or the
+  // pairs' last round would be less than half full: single blocks then, two
+  // workgroups to a CU.  The same bits either way.  Measured at 4 key blocks,
+  // pairs / single (us): 12 heads x 9 query blocks 18.7 / 13.9, x 21 20.5 /
+  // 16.3, x 32 22.5 / 24.2, x 60 41.7 / 37.5, x 66 41.6 / 42.0, x 85 60.7 /
+  // 48.7, x 108 63.2 / 63.7, x 132 79.1 / 75.8.
+  const int64_t cus = cu_count(), pairs = H * ((NQ + 1) / 2), last = pairs % cus;
+  const bool pair = H * NQ > cus && (pairs <= cus || last == 0 || 2 * last >= cus);
+  const auto launch = pair ? launch_bsa<kDirect, kDirect, kDensePair>
+                           : launch_bsa<kDirect, kDirect, kDense>;
+  launch(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride, kv_head_stride, o_tok_stride,
+         o_head_stride, nullptr, nullptr, NK, H, NQ, sm_scale * 1.4426950408889634f, nullptr,
+         nullptr, geo, (hipStream_t)stream, nullptr, nullptr);
   return fvsr_launch_status();
 }
