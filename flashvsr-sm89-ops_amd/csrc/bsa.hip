@@ -311,7 +311,11 @@ FVSR_DEV int64_t query_token(int qb, int qpos, const int32_t* q_map, const WinGe
 // query blocks (waves 0-3 and 4-7) over one K/V stream, so the per-unit
 // start-up and the K/V stream are paid once per two query blocks (2 waves per
 // SIMD, as two 4-wave workgroups would give).
-enum { kSparse = 0, kDense = 1, kDensePair = 2 };
+// kMask: `sel` is the block mask itself, bytes [H, NQ, maxk]; the workgroup
+// compacts its own row into LDS (one load latency, as the index's count and
+// first ids cost), so no index launch precedes the attention: FILL.
+enum { kSparse = 0, kDense = 1, kDensePair = 2, kMask = 3 };
+constexpr int kMaxMask = 4096;  // key blocks a row's LDS list holds (8 KB)
 template <int QM, int KM, int MODE>
 __global__ __attribute__((amdgpu_flat_work_group_size(MODE == kDensePair ? 512 : 256,
                                                       MODE == kDensePair ? 512 : 256),
@@ -325,7 +329,9 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
                     int pieces, float* __restrict__ part) {
   __shared__ __attribute__((aligned(1024))) uint8_t stage0[kStage];
   __shared__ __attribute__((aligned(1024))) uint8_t stage1[kStage];
-  constexpr bool DENSE = MODE != kSparse, PAIR = MODE == kDensePair;
+  constexpr bool DENSE = MODE == kDense || MODE == kDensePair, PAIR = MODE == kDensePair;
+  constexpr bool MASK = MODE == kMask;
+  __shared__ uint16_t kept[MASK ? kMaxMask : 2];
   uint8_t LDS_AS* st0 = (uint8_t LDS_AS*)stage0;
   uint8_t LDS_AS* st1 = (uint8_t LDS_AS*)stage1;
   // Workgroup ids are dispatched round robin over the 8 XCDs; give each XCD a
@@ -349,22 +355,51 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
   const int qb_raw = PAIR ? 2 * up + (wave >> 2) : up;
   const bool q_live = qb_raw < NQ;
   const int qb = q_live ? qb_raw : NQ - 1;
-  int n = DENSE ? (int)maxk : cnt[(int64_t)h * NQ + qb];
-  const int32_t* blocks = DENSE ? nullptr : sel + ((int64_t)h * NQ + qb) * maxk;
+  int n = 0, lo = 0;
+  const int32_t* blocks = nullptr;
+  if constexpr (MASK) {
+    const uint8_t* kr = (const uint8_t*)sel + ((int64_t)h * NQ + qb) * maxk;
+    for (int c0 = 0; c0 < (int)maxk; c0 += 256) {
+      uint32_t f[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) f[u] = c0 + u * 64 + lane < (int)maxk ? kr[c0 + u * 64 + lane] : 0u;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint64_t b = __ballot(f[u] != 0);
+        if (f[u] != 0 && wave == 0)
+          kept[n + __popcll(b & ((1ull << lane) - 1ull))] = (uint16_t)(c0 + u * 64 + lane);
+        n += __popcll(b);
+      }
+    }
+    __syncthreads();
+  } else if constexpr (DENSE) {
+    n = (int)maxk;
+  } else {
+    n = cnt[(int64_t)h * NQ + qb];
+    blocks = sel + ((int64_t)h * NQ + qb) * maxk;
+  }
+  // Kept key block i of this workgroup's part, i < n.
+  const auto block_at = [&](int i) {
+    if constexpr (MASK) return (int)__builtin_amdgcn_readfirstlane((int)kept[lo + i]);
+    if constexpr (DENSE) return i;
+    return blocks[lo + i];
+  };
   // The first two block ids load together with the count (the row holds maxk
   // entries; those past the count are unspecified and then unused), so the
   // first K/V addresses wait for one memory round trip, not two.
   int b0 = 0, b1 = maxk > 1 ? 1 : 0;
-  if (!DENSE && maxk > 0) {
+  if (MODE == kSparse && maxk > 0) {
     b0 = blocks[0];
     b1 = blocks[maxk > 1 ? 1 : 0];
   }
   if (is_piece) {
-    const int pc = slot % pieces, lo = n * pc / pieces;
+    const int pc = slot % pieces;
+    lo = n * pc / pieces;
     n = n * (pc + 1) / pieces - lo;
-    blocks += lo;
-    if (n > 0) b0 = blocks[0];
-    if (n > 1) b1 = blocks[1];
+  }
+  if (is_piece || MASK) {
+    if (n > 0) b0 = block_at(0);
+    if (n > 1) b1 = block_at(1);
   }
   const StepCtx c{2 * n, wave, lane, half, lane >> 4, lane & 15, scale_log2};
   Stream st;
@@ -414,7 +449,7 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
   for (int b = 0; b < n; ++b) {  // two 64-key halves per kept block
     // The block after next loads under this block's steps (a full wait opens
     // every step) and becomes st.blk[1] when the block moves on.
-    const int ahead = DENSE ? (b + 2 < n ? b + 2 : n - 1) : blocks[b + 2 < n ? b + 2 : n - 1];
+    const int ahead = block_at(b + 2 < n ? b + 2 : n - 1);
     bsa_step<KM, NW>(st0, st1, 2 * b, c, st, qf, acc, m_run, l_run);
     bsa_step<KM, NW>(st1, st0, 2 * b + 1, c, st, qf, acc, m_run, l_run);
     st.blk[0] = st.blk[1];
@@ -713,6 +748,32 @@ extern "C" int fvsr_bsa_fwd_ws(const void* q, const void* k, const void* v, void
                                  kv_head_stride, o_tok_stride, o_head_stride, sel, cnt, maxk, H,
                                  NQ, scale_log2, nullptr, nullptr, geo, (hipStream_t)stream, &sp,
                                  workspace);
+  return fvsr_launch_status();
+}
+
+extern "C" int fvsr_bsa_fwd_mask(const void* q, const void* k, const void* v, void* o,
+                                 int64_t q_tok_stride, int64_t q_head_stride,
+                                 int64_t kv_tok_stride, int64_t kv_head_stride,
+                                 int64_t o_tok_stride, int64_t o_head_stride, const uint8_t* keep,
+                                 int64_t H, int64_t NQ, int64_t NK, int64_t head_dim,
+                                 float sm_scale, float* workspace, int64_t workspace_floats,
+                                 void* stream) {
+  if (H < 0 || NQ < 0 || NK < 0) return FVSR_EINVAL;
+  if (H * NQ == 0) return FVSR_OK;
+  static const int32_t kNone = 0;  // no counts are read
+  int rc = bsa_args_ok(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride, kv_head_stride,
+                       o_tok_stride, o_head_stride, (const int32_t*)keep, &kNone, head_dim, H, NQ);
+  if (rc != FVSR_OK) return rc;
+  if (NK > kMaxMask) return FVSR_EUNSUPPORTED;
+  Split sp;
+  rc = split_for(H, NQ, NK, workspace, workspace_floats, sp);
+  if (rc != FVSR_OK) return rc;
+  const WinGeo geo{0, 0, 1, 1};
+  launch_bsa<kDirect, kDirect, kMask>(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride,
+                                      kv_head_stride, o_tok_stride, o_head_stride,
+                                      (const int32_t*)keep, nullptr, NK, H, NQ,
+                                      sm_scale * 1.4426950408889634f, nullptr, nullptr, geo,
+                                      (hipStream_t)stream, &sp, workspace);
   return fvsr_launch_status();
 }
 

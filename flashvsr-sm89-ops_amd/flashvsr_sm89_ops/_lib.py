@@ -70,6 +70,8 @@ _SIGS = {
     "fvsr_bsa_workspace_floats": ([_I64, _I64, _I64], _I64),
     "fvsr_bsa_fwd_ws": ([_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _I64, _I64,
                          _I64, _I64, _I64, _F, _P, _P, _P, _I64, _P], _I),
+    "fvsr_bsa_fwd_mask": ([_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P, _I64, _I64,
+                           _I64, _I64, _F, _P, _I64, _P], _I),
     "fvsr_bsa_fwd_window_ws": ([_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _I64,
                                 _I64, _I64, _I64, _I64, _F, _I64, _I64, _I64, _I, _P, _I64, _P],
                                _I),

@@ -28,6 +28,16 @@ from .. import _lib
 BLOCK = 128
 
 
+_MASK_MAX = 4096  # key blocks per row that fvsr_bsa_fwd_mask takes
+
+
+def _mask_bytes(keep: torch.Tensor) -> torch.Tensor:
+    """keep as contiguous bytes (a bool mask is already one byte per entry: no
+    conversion kernel)."""
+    return (keep.contiguous().view(torch.uint8) if keep.dtype == torch.bool
+            else keep.to(torch.uint8).contiguous())
+
+
 def block_index(keep: torch.Tensor):
     """keep [H, NQ, NK] bool -> (sel [H, NQ, NK] int32, cnt [H, NQ] int32, NK):
     each row of sel holds the kept block ids ascending, then the others
@@ -35,9 +45,7 @@ def block_index(keep: torch.Tensor):
     untrimmed, so nothing is read back to the host."""
     _lib.require_gpu(keep)
     H, NQ, NK = keep.shape
-    # a bool mask is already one byte per entry: no conversion kernel
-    k8 = (keep.contiguous().view(torch.uint8) if keep.dtype == torch.bool
-          else keep.to(torch.uint8).contiguous())
+    k8 = _mask_bytes(keep)
     sel = torch.empty((H, NQ, max(NK, 1)), dtype=torch.int32, device=keep.device)
     cnt = torch.empty((H, NQ), dtype=torch.int32, device=keep.device)
     _lib.check(_lib.lib().fvsr_block_index(k8.data_ptr(), H, NQ, NK, sel.data_ptr(),
@@ -116,11 +124,19 @@ def block_sparse_attention_strided(q, k, v, keep, sm_scale=None, *, heads: int, 
         if kv_raster and NK != NQ:
             raise ValueError("raster-order k/v need as many key blocks as query blocks")
     _lib.require_gpu(q, k, v, out, q_map, kv_map)
-    sel, cnt, maxk = block_index(keep) if index is None else index
+    # A mask in direct order goes to the kernel as it is; else through an index.
+    masked = index is None and window is None and q_map is None and kv_map is None \
+        and 0 < NK <= _MASK_MAX
+    if masked:
+        _lib.require_gpu(keep)
+        maxk = max(NK, 1)
+    else:
+        sel, cnt, maxk = block_index(keep) if index is None else index
     if H != heads:
         raise ValueError(f"block mask has {H} heads, tensors have {heads}")
-    _lib.require_gpu(sel, cnt)
-    _check_index(sel, cnt, maxk, H, NQ)
+    if not masked:
+        _lib.require_gpu(sel, cnt)
+        _check_index(sel, cnt, maxk, H, NQ)
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(head_dim)
     if out is None:
@@ -149,6 +165,15 @@ def block_sparse_attention_strided(q, k, v, keep, sm_scale=None, *, heads: int, 
         _check_extent(out, NQ * BLOCK, *o_strides, heads, head_dim, "out")
         _check_extent(k, NK * BLOCK, *kv_strides, heads, head_dim, "k")
         _check_extent(v, NK * BLOCK, *kv_strides, heads, head_dim, "v")
+        if masked:
+            k8 = _mask_bytes(keep)
+            rc = _lib.lib().fvsr_bsa_fwd_mask(
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), q_strides[0],
+                q_strides[1], kv_strides[0], kv_strides[1], o_strides[0], o_strides[1],
+                k8.data_ptr(), H, NQ, NK, head_dim, float(sm_scale), _lib.ptr(ws), ws_n,
+                _lib.stream(q))
+            _lib.check(rc, "block_sparse_attention")
+            return out
     else:
         for m, n, want in ((q_map, "q_map", NQ * BLOCK), (kv_map, "kv_map", NK * BLOCK)):
             _lib.require_dtype(m, torch.int32, "token map")

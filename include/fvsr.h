@@ -380,6 +380,14 @@ int fvsr_bsa_fwd_ws(const void* q, const void* k, const void* v, void* o, int64_
                     int64_t head_dim, float sm_scale, const int32_t* q_map,
                     const int32_t* kv_map, float* workspace, int64_t workspace_floats,
                     void* stream);
+/* The direct-order call on the block mask itself: keep bytes [H, NQ, NK]
+ * (nonzero = kept), NK at most 4096 (FVSR_EUNSUPPORTED beyond); the results of
+ * fvsr_block_index and fvsr_bsa_fwd_ws, without an index. */
+int fvsr_bsa_fwd_mask(const void* q, const void* k, const void* v, void* o, int64_t q_tok_stride,
+                      int64_t q_head_stride, int64_t kv_tok_stride, int64_t kv_head_stride,
+                      int64_t o_tok_stride, int64_t o_head_stride, const uint8_t* keep, int64_t H,
+                      int64_t NQ, int64_t NK, int64_t head_dim, float sm_scale, float* workspace,
+                      int64_t workspace_floats, void* stream);
 int fvsr_bsa_fwd_window_ws(const void* q, const void* k, const void* v, void* o,
                            int64_t q_tok_stride, int64_t q_head_stride, int64_t kv_tok_stride,
                            int64_t kv_head_stride, int64_t o_tok_stride, int64_t o_head_stride,

@@ -130,3 +130,28 @@ def test_workspace_checks():
     assert L.fvsr_bsa_fwd_ws(*args, ws.data_ptr() + 4, n, _lib.stream(t)) == _lib.FVSR_EUNSUPPORTED
     for units in ((12, 132, 132), (12, 64, 128), (12, 39, 78), (0, 4, 4), (4, 9, 7)):
         assert _plan(*units) == 0
+
+
+@pytest.mark.parametrize("case", [(1, 1, 1), (2, 3, 63), (2, 5, 64), (1, 4, 257), (3, 2, 600),
+                                  (12, 22, 22)])
+def test_mask_equals_index(case):
+    """A mask given as it is against the same mask through block_index, bit
+    for bit: rows of every length around a wave's 64 and a trip's 256 blocks,
+    empty and full rows, other types and layouts of the mask."""
+    from flashvsr_sm89_ops.lcsa.hip_lcsa import block_index, block_sparse_attention_strided
+    H, NQ, NK = case
+    HD = H * 128
+    g = torch.Generator(device=DEV).manual_seed(NK)
+    q, k, v = (torch.randn(n * 128, HD, generator=g, device=DEV).bfloat16() for n in (NQ, NK, NK))
+    keep = torch.rand(H, NQ, NK, generator=g, device=DEV) < 0.3
+    keep[0, 0] = False
+    keep[H - 1, NQ - 1] = True
+    wide = torch.zeros(H, NQ, 2 * NK, dtype=torch.bool, device=DEV)
+    wide[..., ::2] = keep
+    kw = dict(heads=H, head_dim=128, q_strides=(HD, 128), kv_strides=(HD, 128))
+    want = torch.empty_like(q)
+    block_sparse_attention_strided(q, k, v, None, None, out=want, index=block_index(keep), **kw)
+    for m in (keep, keep.to(torch.uint8) * 3, keep.float(), wide[..., ::2]):
+        got = torch.full_like(q, 5.0)
+        block_sparse_attention_strided(q, k, v, m, None, out=got, **kw)
+        assert torch.equal(got, want)
