@@ -50,16 +50,21 @@ FVSR_DEV int k_swz(int r, int c) { return c ^ (r & 15); }
 // half-wave read adjacent 32-byte column blocks; this spreads them over 64 banks.
 FVSR_DEV int v_swz(int r, int c) { return c ^ ((r & 3) << 2); }
 
-// Per-lane state of the K/V stream.  Each wave issues 8 direct loads of 1 KB
-// (4 rows of 256 bytes) per 64-key half: load t covers rows 4*seg .. 4*seg+3
-// of the tile, seg = (wave & 1) * 8 + t, lane i landing at row 4*seg + i/16,
-// physical chunk i%16 and fetching the logical chunk that belongs there.
-// Waves 0-1 stream K, waves 2-3 stream V.  The chunk a lane fetches depends
-// only on t % 4 (K) or not at all (V), so `lbase[t % 4]` (the tile base
-// pointer plus the chunk offset) is fixed for the whole kernel, and a load's
-// address is lbase + token row * row stride: one multiply-add per load.
-// With a token map the 8 rows' tokens of the next-but-one half are gathered
-// one step ahead, so no load ever waits on the map.
+// The K/V stream.  Each wave issues 8 direct loads of 1 KB (4 rows of 256
+// bytes) per 64-key half: load t covers rows 4*seg .. 4*seg+3 of the tile, seg =
+// (wave & 1) * 8 + t, lane i landing at row 4*seg + i/16, physical chunk i%16
+// and fetching the logical chunk that belongs there.  Waves 0-1 stream K,
+// waves 2-3 stream V.  An address is a uniform base (tensor and head, block,
+// half, row group: scalar arithmetic) plus the lane's 32-bit offset (row within
+// the group and chunk), which depends only on t % 4 (K) or not at all (V) and is
+// fixed for the whole kernel: no vector instruction per load.  The VALU is what
+// the softmax and the other workgroup's MFMAs wait for: with a 64-bit address
+// formed per lane and load (eight v_mad_u64_u32 a step) 12 heads x 132 x 132
+// blocks took 562 us against 535, 66 x 198 910 against 871, the C5 layout (a
+// raster qkv tensor read in window order) 568 against 528.
+// With a token map rows are anywhere, so their addresses are formed per lane:
+// the 8 rows' tokens of the next-but-one half are gathered one step ahead, so
+// no load ever waits on the map.
 // How a block position (block id, row within the block) becomes a stored
 // token row: kDirect the position itself; kMap an int32 map gathered from
 // memory; kWin the (2, 8, 8) window partition of a raster-order latent grid
@@ -86,13 +91,15 @@ FVSR_DEV int win_slot(int s, const WinGeo& g) {
 }
 
 struct Stream {
-  const uint8_t* lbase[4];
+  const uint8_t* base;      // the wave's tensor, at its head
+  uint32_t loff[4];         // this lane's offset of load t, at t % 4 (kMap: the chunk only)
+  uint64_t row[8];          // uniform byte offset of load t's first row in half 0 (not kMap)
+  uint64_t hstep;           // ... from half 0 to half 1
+  uint64_t blkoff[2];       // ... of blk[]'s first rows
   uint32_t ts2;             // token row stride in bytes
   const int32_t* kv_map;
   int blk[2];               // key blocks of the current and the next block step
   int tok[8];               // kMap: tokens of the rows of the next half to issue
-  uint32_t woff[8];         // kWin: byte offsets of this lane's rows in half 0
-  uint32_t hw2;             // kWin: bytes from half 0 to half 1 (the next frame)
   WinGeo geo;
 };
 
@@ -115,27 +122,35 @@ FVSR_DEV void gather_tokens(Stream& s, int blk, int hf, int wave, int lane) {
   }
 }
 
-// Token rows are non-negative and below 2^31, so a load's address is one
-// 32 x 32 -> 64-bit multiply-add onto the lane's base pointer (kWin: the
-// window's first row, uniform, plus the lane's 32-bit offset).
+// First 4-row group of load t: 0 .. 15 within a half tile.
+template <int NW>
+FVSR_DEV int stream_seg(int wave, int t) {
+  return (wave % (NW / 2)) * (32 / NW) + t;
+}
+
+// Byte offset of key block blk's first row.
+template <int KM>
+FVSR_DEV uint64_t block_off(const Stream& s, int blk) {
+  return (uint64_t)(KM == kWin ? win_base(blk, s.geo) : (int64_t)blk * kBlk) * s.ts2;
+}
+
+// Stream half hf of key block s.blk[cur].  Token rows of a map are
+// non-negative and below 2^31.
 template <int KM, int NW>
-FVSR_DEV void issue_half(uint8_t LDS_AS* stage, const Stream& s, int blk, int hf, int wave,
-                         int lane) {
+FVSR_DEV void issue_half(uint8_t LDS_AS* stage, Stream& s, int cur, int hf, int wave) {
   uint8_t LDS_AS* tile = stage + (wave >= NW / 2 ? kTile : 0);
-  const uint32_t p0 = KM == kDirect ? (uint32_t)half_pos(blk, hf) : 0u;
-  const uint64_t wb = KM == kWin ? (uint64_t)win_base(blk, s.geo) * s.ts2 + hf * s.hw2 : 0u;
+  const uint8_t* hb = s.base + (KM == kMap ? 0u : s.blkoff[cur] + (hf ? s.hstep : 0u));
+  // Opaque here, so that the compiler widens the offsets beside the loads and
+  // uses their scalar-base form (widened ahead of the loop, each load adds two
+  // 64-bit vectors first: 570 us against 551 at 12 x 132 x 132 blocks).
+  if (KM != kMap)
+    asm volatile("" : "+v"(s.loff[0]), "+v"(s.loff[1]), "+v"(s.loff[2]), "+v"(s.loff[3]));
 #pragma unroll
   for (int t = 0; t < 32 / NW; ++t) {
-    const int seg = (wave % (NW / 2)) * (32 / NW) + t;
-    const uint8_t* src;
-    if (KM == kWin) {
-      src = s.lbase[t & 3] + wb + s.woff[t];
-    } else {
-      const uint32_t row =
-          KM == kMap ? (uint32_t)s.tok[t] : p0 + (uint32_t)stream_row<NW>(wave, t, lane);
-      src = s.lbase[t & 3] + (uint64_t)row * s.ts2;
-    }
-    __builtin_amdgcn_global_load_lds(src, (void LDS_AS*)(tile + seg * 1024), 16, 0, 0);
+    const uint8_t* src = KM == kMap ? hb + (uint64_t)(uint32_t)s.tok[t] * s.ts2 + s.loff[t & 3]
+                                    : hb + s.row[t] + s.loff[t & 3];
+    __builtin_amdgcn_global_load_lds(src, (void LDS_AS*)(tile + stream_seg<NW>(wave, t) * 1024),
+                                     16, 0, 0);
   }
 }
 
@@ -199,7 +214,7 @@ FVSR_DEV void bsa_step(uint8_t LDS_AS* cur, uint8_t LDS_AS* nxt, int it, const S
   // Step it+1 is the second half of this block (it even) or the first half of
   // the next; step it+2 the first or second half of the next block.
   const int hf = it & 1;
-  if (it + 1 < c.steps) issue_half<KM, NW>(nxt, st, st.blk[hf], hf ^ 1, c.wave, c.lane);
+  if (it + 1 < c.steps) issue_half<KM, NW>(nxt, st, hf, hf ^ 1, c.wave);
   if (KM == kMap && it + 2 < c.steps) gather_tokens<KM, NW>(st, st.blk[1], hf, c.wave, c.lane);
   const uint8_t LDS_AS* kt = cur;
   const uint8_t LDS_AS* vt = cur + kTile;
@@ -313,7 +328,9 @@ FVSR_DEV int64_t query_token(int qb, int qpos, const int32_t* q_map, const WinGe
 // SIMD, as two 4-wave workgroups would give).
 // kMask: `sel` is the block mask itself, bytes [H, NQ, maxk]; the workgroup
 // compacts its own row into LDS (one load latency, as the index's count and
-// first ids cost), so no index launch precedes the attention: FILL.
+// first ids cost), so no index launch precedes the attention (a call that
+// built the index -> from the mask, us: 4 heads x 4 x 8 blocks 24.0 -> 14.9,
+// 12 x 9 x 36 42.5 -> 40.7, 12 x 132 x 132 590 -> 586).
 enum { kSparse = 0, kDense = 1, kDensePair = 2, kMask = 3 };
 constexpr int kMaxMask = 4096;  // key blocks a row's LDS list holds (8 KB)
 template <int QM, int KM, int MODE>
@@ -404,27 +421,32 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
   const StepCtx c{2 * n, wave, lane, half, lane >> 4, lane & 15, scale_log2};
   Stream st;
   {
-    const uint16_t* base = (wave >= NW / 2 ? v : k) + (int64_t)h * kv_hs;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int r = stream_row<NW>(wave, t, lane), p = lane & 15;
-      st.lbase[t] = (const uint8_t*)(base + (wave >= NW / 2 ? v_swz(r, p) : k_swz(r, p)) * 8);  // involutions
-    }
+    st.base = (const uint8_t*)((wave >= NW / 2 ? v : k) + (int64_t)h * kv_hs);
     st.ts2 = (uint32_t)(kv_ts * 2);
     st.kv_map = kv_map;
     st.geo = geo;
-    if (KM == kWin) {
-      st.hw2 = (uint32_t)geo.HW * st.ts2;
 #pragma unroll
-      for (int t = 0; t < 32 / NW; ++t)
-        st.woff[t] = (uint32_t)win_slot(stream_row<NW>(wave, t, lane), geo) * st.ts2;
+    for (int t = 0; t < 4; ++t) {
+      const int r = stream_row<NW>(wave, t, lane), p = lane & 15;
+      st.loff[t] = (wave >= NW / 2 ? v_swz(r, p) : k_swz(r, p)) * 16 +  // involutions
+                   (KM == kMap ? 0 : (lane >> 4) * st.ts2);
+    }
+    if (KM != kMap) {
+#pragma unroll
+      for (int t = 0; t < 32 / NW; ++t) {
+        const int r = 4 * stream_seg<NW>(wave, t);
+        st.row[t] = (uint64_t)(KM == kWin ? win_slot(r, geo) : r) * st.ts2;
+      }
+      st.hstep = (uint64_t)(KM == kWin ? geo.HW : kHalf) * st.ts2;
     }
   }
   if (n > 0) {
     st.blk[0] = b0;
     st.blk[1] = n > 1 ? b1 : b0;
+    st.blkoff[0] = block_off<KM>(st, st.blk[0]);
+    st.blkoff[1] = block_off<KM>(st, st.blk[1]);
     gather_tokens<KM, NW>(st, st.blk[0], 0, wave, lane);
-    issue_half<KM, NW>(st0, st, st.blk[0], 0, wave, lane);
+    issue_half<KM, NW>(st0, st, 0, 0, wave);
     gather_tokens<KM, NW>(st, st.blk[0], 1, wave, lane);
   }
 
@@ -454,6 +476,11 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
     bsa_step<KM, NW>(st1, st0, 2 * b + 1, c, st, qf, acc, m_run, l_run);
     st.blk[0] = st.blk[1];
     st.blk[1] = ahead;
+    // A window's first row takes two divisions: formed here, behind the MFMAs,
+    // once per block, not at the head of each step that loads from it (C5
+    // 586 -> 573 us).
+    st.blkoff[0] = st.blkoff[1];
+    st.blkoff[1] = block_off<KM>(st, ahead);
   }
 
   const auto lsw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run),
@@ -690,11 +717,14 @@ void launch_bsa(const void* q, const void* k, const void* v, void* o, int64_t q_
 int bsa_args_ok(const void* q, const void* k, const void* v, const void* o, int64_t q_ts,
                 int64_t q_hs, int64_t kv_ts, int64_t kv_hs, int64_t o_ts, int64_t o_hs,
                 const int32_t* sel, const int32_t* cnt, int64_t head_dim, int64_t H,
-                int64_t NQ) {
+                int64_t NQ, bool mapped = false) {
   if (!q || !k || !v || !o || !sel || !cnt) return FVSR_EINVAL;
   if (head_dim != kD) return FVSR_EUNSUPPORTED;
   // 16-byte rows: token strides and head offsets must keep every row aligned.
   if ((q_ts | q_hs | kv_ts | kv_hs) % 8) return FVSR_EUNSUPPORTED;
+  // Lane offsets of the K/V stream are 32-bit: three rows and a row's bytes
+  // (token maps address whole rows).
+  if (!mapped && 6 * kv_ts + 2 * kD > 0xffffffffLL) return FVSR_EUNSUPPORTED;
   if ((o_ts | o_hs) % 4) return FVSR_EUNSUPPORTED;
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || ((uintptr_t)o & 7)) return FVSR_EUNSUPPORTED;
   if (H * NQ > 0x7fffffff || NQ > 0x7fffffff) return FVSR_EUNSUPPORTED;
@@ -731,7 +761,7 @@ extern "C" int fvsr_bsa_fwd_ws(const void* q, const void* k, const void* v, void
   if (H < 0 || NQ < 0 || NK < 0 || maxk < 0) return FVSR_EINVAL;
   if (H * NQ == 0) return FVSR_OK;
   int rc = bsa_args_ok(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride, kv_head_stride,
-                       o_tok_stride, o_head_stride, sel, cnt, head_dim, H, NQ);
+                       o_tok_stride, o_head_stride, sel, cnt, head_dim, H, NQ, q_map != nullptr);
   if (rc != FVSR_OK) return rc;
   if ((q_map == nullptr) != (kv_map == nullptr)) return FVSR_EUNSUPPORTED;
   Split sp;
