@@ -1212,17 +1212,19 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // other (or two side by side at half speed each), so a tile shape costs
 // rounds = ceil(tiles / CUs) times the clocks of one tile per 128 bytes of K:
 // what its LDS traffic takes at 128 bytes per clock (fragment reads plus the
-// loads' writes) for the tiles up to 128 x 256, its MFMAs (64 clocks each) for
-// the larger ones; 192 rows pay 8% for their larger share of loads (17% at
-// long K, where the 256-row kernel prefetches into L2).  Equal costs go to the
-// larger tile.  Over 24 shapes (M 100-18432, N 1536-8960, K 1536 and 8960) the
-// choice is within 4% of the fastest of the eight.
+// loads' writes) up to 128 x 128, its MFMAs (64 clocks each) at 256 x 256.  The
+// two between are priced as measured: 192 rows at 1.17 of their MFMAs (1.22 at
+// long K, where the 256-row kernel prefetches into L2); 128 x 256 at 1.25 of
+// its LDS traffic, 1.07 at long K, where its start and epilogue weigh less.
+// Equal costs go to the larger tile.  Over 26 shapes (M 1300-15000, N 1536-8960,
+// K 1536 and 8960) the choice is within 4% of the fastest of the eight.
 // Where lines lie, both sides measured (us): M = 512 (N = K = 1536) 64 x 64
 // 5.5 against 64 x 128 7.1; M = 1152 8.5 / 8.2; M = 2079 128 x 128 11.3
 // against 64 x 128 11.7; M = 2800 ring 128 15.4 against 64 x 128 16.3; 12000
-// rows 192 against 256 32.7 / 35.4; 9000 rows 31.0 / 22.7.  At long K the
-// 128 x 256 tile of gemm_fp8_small (three slots, 4000 rows 50.5) replaces the
-// ring's (two, 59.4); at K = 1536 its longer start costs more (16.5 / 15.3).
+// rows 192 against 256 32.7 / 35.4; 9000 rows 31.0 / 22.7; three rounds of 256
+// rows against five of 128 (4227 x 8960) 59.4 / 66.8.  At long K the 128 x 256
+// tile of gemm_fp8_small (three slots, 4000 rows 50.5) replaces the ring's
+// (two, 59.4); at K = 1536 its longer start costs more (16.5 / 15.3).
 Plan plan_gemm(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int epilogue,
                bool direct) {
   struct Option {
@@ -1231,8 +1233,8 @@ Plan plan_gemm(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int ep
   };
   static constexpr Option kOptions[] = {
       {Path::kRing256, 256, 256, 2048, 2048}, {Path::kRing, 256, 256, 2048, 2048},
-      {Path::kRing192, 192, 256, 1664, 1792}, {Path::kRing128, 128, 256, 1152, 1152},
-      {Path::k128x256, 128, 256, 1152, 1152}, {Path::k128x128, 128, 128, 768, 768},
+      {Path::kRing192, 192, 256, 1800, 1880}, {Path::kRing128, 128, 256, 1440, 1440},
+      {Path::k128x256, 128, 256, 1440, 1230}, {Path::k128x128, 128, 128, 768, 768},
       {Path::k64x128, 64, 128, 576, 576},     {Path::k64x64, 64, 64, 384, 384},
   };
   // Every row offset of either operand within 32 bits; the ring takes K in
