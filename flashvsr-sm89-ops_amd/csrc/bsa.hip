@@ -68,8 +68,14 @@ FVSR_DEV int v_swz(int r, int c) { return c ^ ((r & 3) << 2); }
 // How a block position (block id, row within the block) becomes a stored
 // token row: kDirect the position itself; kMap an int32 map gathered from
 // memory; kWin the (2, 8, 8) window partition of a raster-order latent grid
-// (WindowPartition3D, reference integrate.py:70-94), in closed form.
-enum { kDirect = 0, kMap = 1, kWin = 2 };
+// (WindowPartition3D, reference integrate.py:70-94), in closed form; kFar
+// (K/V only) the position itself, as kDirect, for rows so far apart that a
+// lane's offset (three rows) leaves 32 bits: its addresses are formed per lane,
+// as a map's are.
+enum { kDirect = 0, kMap = 1, kWin = 2, kFar = 3 };
+constexpr bool per_lane(int km) { return km == kMap || km == kFar; }
+// Largest K/V token stride, in elements, of the fixed lane offsets.
+constexpr int64_t kNearStride = (0xffffffffLL - 2 * kD) / 6;
 
 // Latent grid of the kWin mode: row width W and frame size HW in tokens;
 // windows per row nww = W / 8 and per frame pair nwhw = (H / 8) * nww.
@@ -92,14 +98,14 @@ FVSR_DEV int win_slot(int s, const WinGeo& g) {
 
 struct Stream {
   const uint8_t* base;      // the wave's tensor, at its head
-  uint32_t loff[4];         // this lane's offset of load t, at t % 4 (kMap: the chunk only)
-  uint64_t row[8];          // uniform byte offset of load t's first row in half 0 (not kMap)
+  uint32_t loff[4];         // this lane's offset of load t, at t % 4 (per_lane: the chunk only)
+  uint64_t row[8];          // uniform byte offset of load t's first row in half 0 (not per_lane)
   uint64_t hstep;           // ... from half 0 to half 1
   uint64_t blkoff[2];       // ... of blk[]'s first rows
   uint32_t ts2;             // token row stride in bytes
   const int32_t* kv_map;
   int blk[2];               // key blocks of the current and the next block step
-  int tok[8];               // kMap: tokens of the rows of the next half to issue
+  int tok[8];               // per_lane: tokens of the rows of the next half to issue
   WinGeo geo;
 };
 
@@ -119,6 +125,10 @@ FVSR_DEV void gather_tokens(Stream& s, int blk, int hf, int wave, int lane) {
     const int64_t p0 = half_pos(blk, hf);
 #pragma unroll
     for (int t = 0; t < 32 / NW; ++t) s.tok[t] = s.kv_map[p0 + stream_row<NW>(wave, t, lane)];
+  } else if (KM == kFar) {
+#pragma unroll
+    for (int t = 0; t < 32 / NW; ++t)
+      s.tok[t] = (int)(half_pos(blk, hf) + stream_row<NW>(wave, t, lane));
   }
 }
 
@@ -139,16 +149,16 @@ FVSR_DEV uint64_t block_off(const Stream& s, int blk) {
 template <int KM, int NW>
 FVSR_DEV void issue_half(uint8_t LDS_AS* stage, Stream& s, int cur, int hf, int wave) {
   uint8_t LDS_AS* tile = stage + (wave >= NW / 2 ? kTile : 0);
-  const uint8_t* hb = s.base + (KM == kMap ? 0u : s.blkoff[cur] + (hf ? s.hstep : 0u));
+  const uint8_t* hb = s.base + (per_lane(KM) ? 0u : s.blkoff[cur] + (hf ? s.hstep : 0u));
   // Opaque here, so that the compiler widens the offsets beside the loads and
   // uses their scalar-base form (widened ahead of the loop, each load adds two
   // 64-bit vectors first: 570 us against 551 at 12 x 132 x 132 blocks).
-  if (KM != kMap)
+  if (!per_lane(KM))
     asm volatile("" : "+v"(s.loff[0]), "+v"(s.loff[1]), "+v"(s.loff[2]), "+v"(s.loff[3]));
 #pragma unroll
   for (int t = 0; t < 32 / NW; ++t) {
-    const uint8_t* src = KM == kMap ? hb + (uint64_t)(uint32_t)s.tok[t] * s.ts2 + s.loff[t & 3]
-                                    : hb + s.row[t] + s.loff[t & 3];
+    const uint8_t* src = per_lane(KM) ? hb + (uint64_t)(uint32_t)s.tok[t] * s.ts2 + s.loff[t & 3]
+                                      : hb + s.row[t] + s.loff[t & 3];
     __builtin_amdgcn_global_load_lds(src, (void LDS_AS*)(tile + stream_seg<NW>(wave, t) * 1024),
                                      16, 0, 0);
   }
@@ -215,7 +225,7 @@ FVSR_DEV void bsa_step(uint8_t LDS_AS* cur, uint8_t LDS_AS* nxt, int it, const S
   // the next; step it+2 the first or second half of the next block.
   const int hf = it & 1;
   if (it + 1 < c.steps) issue_half<KM, NW>(nxt, st, hf, hf ^ 1, c.wave);
-  if (KM == kMap && it + 2 < c.steps) gather_tokens<KM, NW>(st, st.blk[1], hf, c.wave, c.lane);
+  if (per_lane(KM) && it + 2 < c.steps) gather_tokens<KM, NW>(st, st.blk[1], hf, c.wave, c.lane);
   const uint8_t LDS_AS* kt = cur;
   const uint8_t LDS_AS* vt = cur + kTile;
   const int lane = c.lane, half = c.half;
@@ -319,7 +329,7 @@ FVSR_DEV int64_t query_token(int qb, int qpos, const int32_t* q_map, const WinGe
 }
 
 // QM / KM: how query and key/value block positions become stored token rows
-// (kDirect, kMap or kWin, see above); the output rows are the query rows.
+// (kDirect, kMap, kWin or kFar, see above); the output rows are the query rows.
 // kDense: every key block 0..maxk-1 is kept for every query block (the
 // cross-attention over the cached prompt, integrate.py:132-143): no block
 // index is read.  kDensePair: the same with a workgroup of 8 waves taking two
@@ -429,9 +439,9 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
     for (int t = 0; t < 4; ++t) {
       const int r = stream_row<NW>(wave, t, lane), p = lane & 15;
       st.loff[t] = (wave >= NW / 2 ? v_swz(r, p) : k_swz(r, p)) * 16 +  // involutions
-                   (KM == kMap ? 0 : (lane >> 4) * st.ts2);
+                   (per_lane(KM) ? 0 : (lane >> 4) * st.ts2);
     }
-    if (KM != kMap) {
+    if (!per_lane(KM)) {
 #pragma unroll
       for (int t = 0; t < 32 / NW; ++t) {
         const int r = 4 * stream_seg<NW>(wave, t);
@@ -717,14 +727,11 @@ void launch_bsa(const void* q, const void* k, const void* v, void* o, int64_t q_
 int bsa_args_ok(const void* q, const void* k, const void* v, const void* o, int64_t q_ts,
                 int64_t q_hs, int64_t kv_ts, int64_t kv_hs, int64_t o_ts, int64_t o_hs,
                 const int32_t* sel, const int32_t* cnt, int64_t head_dim, int64_t H,
-                int64_t NQ, bool mapped = false) {
+                int64_t NQ) {
   if (!q || !k || !v || !o || !sel || !cnt) return FVSR_EINVAL;
   if (head_dim != kD) return FVSR_EUNSUPPORTED;
   // 16-byte rows: token strides and head offsets must keep every row aligned.
   if ((q_ts | q_hs | kv_ts | kv_hs) % 8) return FVSR_EUNSUPPORTED;
-  // Lane offsets of the K/V stream are 32-bit: three rows and a row's bytes
-  // (token maps address whole rows).
-  if (!mapped && 6 * kv_ts + 2 * kD > 0xffffffffLL) return FVSR_EUNSUPPORTED;
   if ((o_ts | o_hs) % 4) return FVSR_EUNSUPPORTED;
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || ((uintptr_t)o & 7)) return FVSR_EUNSUPPORTED;
   if (H * NQ > 0x7fffffff || NQ > 0x7fffffff) return FVSR_EUNSUPPORTED;
@@ -761,7 +768,7 @@ extern "C" int fvsr_bsa_fwd_ws(const void* q, const void* k, const void* v, void
   if (H < 0 || NQ < 0 || NK < 0 || maxk < 0) return FVSR_EINVAL;
   if (H * NQ == 0) return FVSR_OK;
   int rc = bsa_args_ok(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride, kv_head_stride,
-                       o_tok_stride, o_head_stride, sel, cnt, head_dim, H, NQ, q_map != nullptr);
+                       o_tok_stride, o_head_stride, sel, cnt, head_dim, H, NQ);
   if (rc != FVSR_OK) return rc;
   if ((q_map == nullptr) != (kv_map == nullptr)) return FVSR_EUNSUPPORTED;
   Split sp;
@@ -774,10 +781,10 @@ extern "C" int fvsr_bsa_fwd_ws(const void* q, const void* k, const void* v, void
                            kv_head_stride, o_tok_stride, o_head_stride, sel, cnt, maxk, H, NQ,
                            scale_log2, q_map, kv_map, geo, (hipStream_t)stream, &sp, workspace);
   else
-    launch_bsa<kDirect, kDirect>(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride,
-                                 kv_head_stride, o_tok_stride, o_head_stride, sel, cnt, maxk, H,
-                                 NQ, scale_log2, nullptr, nullptr, geo, (hipStream_t)stream, &sp,
-                                 workspace);
+    (kv_tok_stride <= kNearStride ? launch_bsa<kDirect, kDirect> : launch_bsa<kDirect, kFar>)(
+        q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride, kv_head_stride, o_tok_stride,
+        o_head_stride, sel, cnt, maxk, H, NQ, scale_log2, nullptr, nullptr, geo,
+        (hipStream_t)stream, &sp, workspace);
   return fvsr_launch_status();
 }
 
@@ -799,11 +806,11 @@ extern "C" int fvsr_bsa_fwd_mask(const void* q, const void* k, const void* v, vo
   rc = split_for(H, NQ, NK, workspace, workspace_floats, sp);
   if (rc != FVSR_OK) return rc;
   const WinGeo geo{0, 0, 1, 1};
-  launch_bsa<kDirect, kDirect, kMask>(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride,
-                                      kv_head_stride, o_tok_stride, o_head_stride,
-                                      (const int32_t*)keep, nullptr, NK, H, NQ,
-                                      sm_scale * 1.4426950408889634f, nullptr, nullptr, geo,
-                                      (hipStream_t)stream, &sp, workspace);
+  (kv_tok_stride <= kNearStride ? launch_bsa<kDirect, kDirect, kMask>
+                                : launch_bsa<kDirect, kFar, kMask>)(
+      q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride, kv_head_stride, o_tok_stride,
+      o_head_stride, (const int32_t*)keep, nullptr, NK, H, NQ, sm_scale * 1.4426950408889634f,
+      nullptr, nullptr, geo, (hipStream_t)stream, &sp, workspace);
   return fvsr_launch_status();
 }
 
@@ -850,10 +857,10 @@ extern "C" int fvsr_bsa_fwd_window_ws(const void* q, const void* k, const void* 
                            o_tok_stride, o_head_stride, sel, cnt, maxk, H, NQ, scale_log2,
                            nullptr, nullptr, geo, (hipStream_t)stream, &sp, workspace);
   else
-    launch_bsa<kWin, kDirect>(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride,
-                              kv_head_stride, o_tok_stride, o_head_stride, sel, cnt, maxk, H, NQ,
-                              scale_log2, nullptr, nullptr, geo, (hipStream_t)stream, &sp,
-                              workspace);
+    (kv_tok_stride <= kNearStride ? launch_bsa<kWin, kDirect> : launch_bsa<kWin, kFar>)(
+        q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride, kv_head_stride, o_tok_stride,
+        o_head_stride, sel, cnt, maxk, H, NQ, scale_log2, nullptr, nullptr, geo,
+        (hipStream_t)stream, &sp, workspace);
   return fvsr_launch_status();
 }
 
@@ -894,8 +901,9 @@ extern "C" int fvsr_attn_dense(const void* q, const void* k, const void* v, void
   // 48.7, x 108 63.2 / 63.7, x 132 79.1 / 75.8.
   const int64_t cus = cu_count(), pairs = H * ((NQ + 1) / 2), last = pairs % cus;
   const bool pair = H * NQ > cus && (pairs <= cus || last == 0 || 2 * last >= cus);
-  const auto launch = pair ? launch_bsa<kDirect, kDirect, kDensePair>
-                           : launch_bsa<kDirect, kDirect, kDense>;
+  const auto launch = kv_tok_stride > kNearStride ? launch_bsa<kDirect, kFar, kDense>
+                      : pair                      ? launch_bsa<kDirect, kDirect, kDensePair>
+                                                  : launch_bsa<kDirect, kDirect, kDense>;
   launch(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride, kv_head_stride, o_tok_stride,
          o_head_stride, nullptr, nullptr, NK, H, NQ, sm_scale * 1.4426950408889634f, nullptr,
          nullptr, geo, (hipStream_t)stream, nullptr, nullptr);

@@ -325,8 +325,7 @@ int fvsr_draft_block_mask(const void* q, int64_t q_tok_stride, const int32_t* q_
  * and query block i, softmax(Q_i K_J^T * sm_scale) V_J over the kept key
  * blocks J = sel[h,i,0..cnt[h,i]-1]; rows with cnt 0 are written as zeros.
  * q/k/v/o bf16, element (token t, head h, dim d) at ptr[t*tok_stride +
- * h*head_stride + d]; head_dim must be 128; sel row stride is maxk; without
- * maps kv_tok_stride is at most 715827832 elements (1.4 GB a row).
+ * h*head_stride + d]; head_dim must be 128; sel row stride is maxk.
  * tok_map: NULL, or int32 [NQ*128] (queries/outputs) and [NK*128] (keys) maps
  * from block-order position to stored token index (kmap), letting raster-order
  * tensors be read in window order without a copy.

@@ -155,3 +155,40 @@ def test_mask_equals_index(case):
         got = torch.full_like(q, 5.0)
         block_sparse_attention_strided(q, k, v, m, None, out=got, **kw)
         assert torch.equal(got, want)
+
+
+def test_far_rows():
+    """K/V rows further apart than 32-bit lane offsets reach (a token stride of
+    1.4 GB), through each entry: bit for bit the packed tensors' results."""
+    from flashvsr_sm89_ops.lcsa.hip_lcsa import (block_index, block_sparse_attention_strided,
+                                                 dense_attention_strided)
+    stride = 715827840  # the next multiple of 8 below stays with the lane offsets
+    n = 127 * stride + 256
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 2 * n + (8 << 30):
+        pytest.skip("needs 190 GB of free GPU memory")
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q, k, v = (torch.randn(m, 128, generator=g, device=DEV).bfloat16() for m in (256, 128, 128))
+    far = torch.empty(n, dtype=torch.bfloat16, device=DEV)
+    kf, vf = (far.as_strided((128, 128), (stride, 1), c) for c in (0, 128))
+    try:
+        for t in range(128):
+            kf[t] = k[t]
+            vf[t] = v[t]
+        keep = torch.ones(1, 2, 1, dtype=torch.bool, device=DEV)
+        for kw in ({}, {"index": block_index(keep)}, {"index": block_index(keep),
+                                                      "window": (2, 8, 16, False)}, None):
+            got = []
+            for kk, vv, ts in ((k, v, 128), (kf, vf, stride)):
+                out = torch.zeros(256, 128, dtype=torch.bfloat16, device=DEV)
+                args = dict(heads=1, head_dim=128, q_strides=(128, 128), kv_strides=(ts, 128),
+                            out=out)
+                if kw is None:
+                    dense_attention_strided(q, kk, vv, None, **args)
+                else:
+                    block_sparse_attention_strided(q, kk, vv, keep, **args, **kw)
+                got.append(out)
+            assert torch.equal(*got) and bool(got[0].any())
+    finally:
+        del far, kf, vf
+        torch.cuda.empty_cache()
