@@ -777,7 +777,7 @@ OP_KERNELS = {
     "ln_modulate_quant": ("ln_modulate_row<false, true, false>", None),
     "gemm_qkv": ("gemm_fp8_ring<0, true, 4, false>", 240 * 256),
     "rms_rope_qk": ("rms_rope_qk_vec", None),
-    "bsa": ("bsa_fwd_kernel<2, 2, false>", None),
+    "bsa": ("bsa_fwd_kernel<2, 2, 0>", None),
     "quant_attn": ("quant_rows_vec<3, false>", None),
     "gemm_o": ("gemm_fp8_ring<0, true, 4, false>", 200 * 256),
     "gate_add_ln_modulate_quant": ("ln_modulate_row<false, true, true>", None),
