@@ -19,7 +19,8 @@ for gfx950 instead of as a sequence of eager ops:
   gate_add [+ the next block's AdaLN + quant]  (1 pass)
 
 With cross-attention weights (not part of the BASELINE C5 block stack) the
-self-attention's gate_add is followed by norm3 (affine LayerNorm + quant), the
+self-attention's gate_add is followed by norm3 (affine LayerNorm + quant; one
+pass: the rows are read once less, the block 1588 -> 1582 us at 16896 tokens), the
 cross q projection, RMSNorm, dense attention over the cached prompt K/V, the
 o projection, and the residual add fused with the FFN's AdaLN.  Weights use
 per-output-channel scales, activations per-token scales.
@@ -34,7 +35,8 @@ from . import _lib
 from .fp8_ffn import fused_gelu_quant_fp8
 from .fp8_linear import FP8Linear, fp8_gemm
 from .fp8_quant import quantize_fp8, quantize_weight_fp8
-from .fused_adaln import (fused_gate_add, fused_gate_add_ln_modulate_quant,
+from .fused_adaln import (fused_gate_add, fused_gate_add_layer_norm_quant,
+                          fused_gate_add_ln_modulate_quant,
                           fused_ln_modulate_quant)
 from .fused_rms_rope import fused_rms_rope_qk
 from .cross_attn import cross_attention_out, unit_gate
@@ -144,10 +146,11 @@ def dit_block_forward(x: torch.Tensor, wts: DiTBlockWeights, t_mod: torch.Tensor
         x1, x8, xs = fused_gate_add_ln_modulate_quant(x, gate_msa, yo, scale_mlp, shift_mlp, eps)
     else:
         c = wts.cross
-        mark("gate_add")
-        x1 = fused_gate_add(x, gate_msa, yo.view(B, L, D))
+        mark("gate_add_layer_norm_quant")
+        x1, x8, xs = fused_gate_add_layer_norm_quant(x, gate_msa, yo, c["norm3_w"], c["norm3_b"],
+                                                     eps)
         yc = cross_attention_out(x1, c["norm3_w"], c["norm3_b"], c["q"], c["norm_q"], c["k"],
-                                 c["v"], c["o"], heads, eps, hook=hook)
+                                 c["v"], c["o"], heads, eps, hook=hook, x8s=(x8, xs))
         mark("gate_add_ln_modulate_quant")
         x1, x8, xs = fused_gate_add_ln_modulate_quant(x1, unit_gate(D, x.device), yc, scale_mlp,
                                                       shift_mlp, eps)

@@ -73,14 +73,17 @@ def cross_attention_out(x: torch.Tensor, norm3_weight: torch.Tensor,
                         norm3_bias: torch.Tensor | None, q_proj: tuple,
                         norm_q_weight: torch.Tensor, cache_k: torch.Tensor,
                         cache_v: torch.Tensor, o_proj: tuple, num_heads: int,
-                        eps: float = 1e-6, hook=None) -> torch.Tensor:
+                        eps: float = 1e-6, hook=None, x8s=None) -> torch.Tensor:
     """``cross_attn(norm3(x))`` for x [1, L, D] bf16 with per-token activation
     scales: q_proj / o_proj are (e4m3 weight [D, D], weight scale, bias)
-    triples; cache_k / cache_v [1, Lk, D].  Returns the o projection [L, D]."""
+    triples; cache_k / cache_v [1, Lk, D].  ``x8s``: norm3's codes and row
+    scales where the caller has them.  Returns the o projection [L, D]."""
     mark = hook or (lambda name: None)
     B, L, D = x.shape
-    mark("layer_norm_quant")
-    x8, xs = layer_norm_quant(x, norm3_weight, norm3_bias, eps)
+    if x8s is None:
+        mark("layer_norm_quant")
+        x8s = layer_norm_quant(x, norm3_weight, norm3_bias, eps)
+    x8, xs = x8s
     mark("gemm_cross_q")
     q = fp8_gemm(x8, xs, *q_proj).view(B, L, D)
     mark("rms_cross_q")

@@ -146,6 +146,33 @@ def fused_gate_add_layer_norm(x: torch.Tensor, gate: torch.Tensor, residual: tor
     return x1, out
 
 
+def fused_gate_add_layer_norm_quant(x: torch.Tensor, gate: torch.Tensor, residual: torch.Tensor,
+                                    weight: torch.Tensor, bias: torch.Tensor | None,
+                                    eps: float = 1e-6):
+    """x1 = fused_gate_add(x, gate, residual), then layer_norm_quant(x1, weight,
+    bias): (x1, codes [B*L, D] e4m3, row scales [B*L, 1] fp32), the same bits.
+    One pass over the rows where the kernel takes the shape (whole 16-byte
+    chunks, at most 1536 columns), else the two steps."""
+    B, L, D = x.shape
+    res = residual.view(B, L, D)
+    ok = all(t.is_contiguous() and t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0
+             for t in (x, gate, res)) and tuple(gate.shape) == (B, 1, D)
+    if ok and D % 8 == 0 and D <= 1536:
+        _lib.require_gpu(x, res, gate)
+        x2, w, b = _ln_affine_args(x, weight, bias)
+        if w.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0:
+            x1 = torch.empty_like(x2)
+            q = torch.empty((B * L, D), dtype=torch.float8_e4m3fn, device=x.device)
+            s = torch.empty((B * L, 1), dtype=torch.float32, device=x.device)
+            _lib.check(_lib.lib().fvsr_gate_add_layer_norm(
+                x2.data_ptr(), gate.data_ptr(), res.data_ptr(), x1.data_ptr(), w.data_ptr(),
+                b.data_ptr(), None, B, L, D, float(eps), q.data_ptr(), s.data_ptr(),
+                _lib.stream(x2)), "fused_gate_add_layer_norm_quant")
+            return x1, q, s
+    x1 = fused_gate_add(x, gate, res)
+    return (x1, *layer_norm_quant(x1, weight, bias, eps))
+
+
 def layer_norm_quant(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
                      eps: float = 1e-6, write_bf16: bool = False):
     """layer_norm + per-row e4m3 quantisation of its output in one pass.

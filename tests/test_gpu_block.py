@@ -175,6 +175,29 @@ def test_gate_add_layer_norm_fused_equals_separate(B, L, D):
     assert torch.equal(x1, x1r) and torch.equal(y, yr)
 
 
+@pytest.mark.parametrize("B,L,D,off", [(1, 4224, 1536, 0), (2, 33, 1536, 0), (1, 7, 512, 0),
+                                       (3, 5, 768, 0), (1, 5, 1544, 0), (1, 3, 8, 0),
+                                       (2, 7, 512, 4), (1, 4, 100, 0)])
+def test_gate_add_layer_norm_quant_equals_separate(B, L, D, off):
+    """Gated residual + norm3 + codes: the one pass and, where it does not apply
+    (more than 1536 columns, no whole 16-byte chunks, a gate off a 16-byte
+    boundary), the two steps give the bits of fused_gate_add followed by
+    layer_norm_quant."""
+    import flashvsr_sm89_ops as fv
+    from flashvsr_sm89_ops.fused_adaln import fused_gate_add_layer_norm_quant, layer_norm_quant
+    g = torch.Generator().manual_seed(5 * B * L + D)
+    x, r = (torch.randn(B, L, D, generator=g).bfloat16().to(DEV) for _ in range(2))
+    gate = torch.empty(B * D + off, dtype=torch.bfloat16, device=DEV)[off:].view(B, 1, D)
+    gate.copy_(0.3 * torch.randn(B, 1, D, generator=g))
+    w = (1 + 0.1 * torch.randn(D, generator=g)).bfloat16().to(DEV)
+    b = (0.1 * torch.randn(D, generator=g)).bfloat16().to(DEV)
+    x1, q, s = fused_gate_add_layer_norm_quant(x, gate, r.view(B * L, D), w, b, eps=1e-6)
+    x1r = fv.fused_gate_add(x, gate, r)
+    qr, sr = layer_norm_quant(x1r, w, b, eps=1e-6)
+    assert torch.equal(x1, x1r) and torch.equal(s, sr)
+    assert torch.equal(q.view(torch.uint8), qr.view(torch.uint8))
+
+
 @pytest.mark.parametrize("B,L,D", [(1, 4224, 1536), (2, 33, 1536), (1, 7, 512)])
 def test_gate_add_ln_modulate_fused_equals_separate(B, L, D):
     """The fused pass is bit-identical to fused_gate_add followed by
