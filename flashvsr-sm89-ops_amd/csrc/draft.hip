@@ -120,8 +120,8 @@ __global__ __launch_bounds__(kPoolWaves * 64) void pool_kernel(
 // blocks at a time, each lane 8-channel chunks l / 16 + 4 g of its rows, all
 // loads of 128 channels in flight together.  (Dot products by fp64 fmas with
 // the query values broadcast from LDS read the LDS 256 times per key block:
-// 11.5 us at 12 heads x 66 x 198 blocks against 8.4 here.)  Pass 2: wave w takes row l0+w, its maximum, exponentials and sum by
-// wave reductions, and writes the softmax as bf16 bits to attn[h][l0+w][:]
+// 11.5 us at 12 heads x 66 x 198 blocks against 8.4 here.)  Pass 2: wave w
+// takes row l0+w, its maximum, exponentials and sum by wave reductions, and writes the softmax as bf16 bits to attn[h][l0+w][:]
 // and, for the threshold search, the row's histogram of nonzero patterns by
 // high byte to hist[h][l0+w][0..127] (attn <= 1 or the NaN 0x7fc0, so the high
 // byte is below 128).
