@@ -1266,7 +1266,7 @@ Plan plan_gemm(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int ep
     // holds a round more than another (ffn0 2310 tiles: 232 workgroups of 10
     // tiles and fewer instead of 256 of 9 or 10; qkv 240, o and ffn2 200): the
     // critical path is unchanged and the idle CUs' power goes to the others'
-    // clock (ffn0 216 -> 210 us, o 40.8 -> 39.7 us on one box).
+    // clock (ffn0 216 -> 210 us, o 40.8 -> 39.7 us).
     const bool persistent = o.path == Path::kRing || o.path == Path::kRing128 ||
                             o.path == Path::kRing192 || o.path == Path::kRing256;
     best = {o.path, (unsigned)(persistent && tiles > slots ? 8 * cdiv(tiles, 8 * rounds) : tiles)};
