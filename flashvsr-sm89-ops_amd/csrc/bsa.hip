@@ -21,7 +21,9 @@
 //                     V tile through ds_read_b64_tr_b16 (lane i of each
 //                     16-lane group receives element i%4 of the 8 bytes
 //                     addressed by lane 4j + i/4, for j = 0..3).
-// Rows whose block list is empty produce zeros (lcsa/triton_lcsa.py:59-60).
+// Rows whose block list is empty produce zeros (lcsa/triton_lcsa.py:59-60); a
+// logit of -inf weighs 0, and a query all of whose logits are -inf gives NaN, as
+// softmax does.
 #include <algorithm>
 
 #include "common.h"
@@ -316,6 +318,8 @@ FVSR_DEV void bsa_step(uint8_t LDS_AS* cur, uint8_t LDS_AS* nxt, int it, const S
   }
 }
 
+constexpr float kMaxStart = -3.40282347e38f;  // lowest finite float
+
 // Floats of one piece's partial result: O^T of 128 queries x 128 dims, then
 // the queries' running maxima (log2 domain) and sums.
 constexpr int kPieceFloats = kBlk * kD + 2 * kBlk;
@@ -476,7 +480,11 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
   for (int jd = 0; jd < 4; ++jd)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[jd][e] = 0.0f;
-  float m_run = -__builtin_huge_valf(), l_run = 0.0f;
+  // The running maximum (log2 domain) starts at the lowest finite value, not at
+  // -inf: while a query has met only logits of -inf, exponents are -inf and its
+  // sums stay 0 (from -inf they would be -inf - -inf, and the sums NaN for good,
+  // in whichever half block or piece comes first).
+  float m_run = kMaxStart, l_run = 0.0f;
 
   for (int b = 0; b < n; ++b) {  // two 64-key halves per kept block
     // The block after next loads under this block's steps (a full wait opens
@@ -515,7 +523,7 @@ void bsa_fwd_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__
     }
     return;
   }
-  const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+  const float inv = n > 0 ? 1.0f / l_tot : 0.0f;  // only -inf logits: 0 / 0
   if (PAIR) {
     __syncthreads();  // waves 4-7 stage through stage1, which the last step reads
     if (!q_live) return;
@@ -594,9 +602,11 @@ __global__ __launch_bounds__(kThreads) void bsa_combine_kernel(
   for (int s = 0; s < P; ++s)
     if (l[s] != -1.0f) mx = fmaxf(mx, m[s]);
   float lt = 0.0f, acc[16] = {};
+  bool blocks = false;
 #pragma unroll
   for (int s = 0; s < P; ++s) {
     const bool any = s < pieces && l[s] != -1.0f;
+    blocks |= any;
     const float w = any ? __builtin_amdgcn_exp2f(m[s] - mx) : 0.0f;
     lt += any ? w * l[s] : 0.0f;
 #pragma unroll
@@ -604,7 +614,7 @@ __global__ __launch_bounds__(kThreads) void bsa_combine_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[g * 4 + e] += any ? w * v[s][g][e] : 0.0f;
   }
-  const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+  const float inv = blocks ? 1.0f / lt : 0.0f;  // only -inf logits: 0 / 0
 #pragma unroll
   for (int g = 0; g < 4; ++g)
     *(u32x2_t*)(orow + jd * 32 + g * 8 + half * 4) =

@@ -323,7 +323,9 @@ int fvsr_draft_block_mask(const void* q, int64_t q_tok_stride, const int32_t* q_
  * Block-sparse attention over 128-token blocks, reference _bsa_fwd_kernel /
  * block_sparse_attention (lcsa/triton_lcsa.py:19-61,74-94): for each head h
  * and query block i, softmax(Q_i K_J^T * sm_scale) V_J over the kept key
- * blocks J = sel[h,i,0..cnt[h,i]-1]; rows with cnt 0 are written as zeros.
+ * blocks J = sel[h,i,0..cnt[h,i]-1]; rows with cnt 0 are written as zeros.  A
+ * logit of -inf (a masked key: an infinity in k) weighs 0 wherever it lies; a
+ * query whose kept logits are all -inf gives NaN, as softmax over them does.
  * q/k/v/o bf16, element (token t, head h, dim d) at ptr[t*tok_stride +
  * h*head_stride + d]; head_dim must be 128; sel row stride is maxk.
  * tok_map: NULL, or int32 [NQ*128] (queries/outputs) and [NK*128] (keys) maps
