@@ -30,6 +30,7 @@
 #include <utility>
 
 #include "common.h"
+#include "small_tile.h"
 
 // Buffer loads straight into LDS (buffer_load_dwordx4 ... lds): the 16 bytes
 // at base + voffset + soffset of every lane land at M0 + 16 * lane.
@@ -856,18 +857,6 @@ FVSR_DEV void small_sched(std::integer_sequence<int, Q...>) {
   (small_slot<LOADS, NM, NL, ND, Q>(), ...);
 }
 
-// Tile of TM = 64 * MJ rows by TN = 64 * NI columns; each of the 4 waves owns
-// a 32 * MJ by 32 * NI quadrant.  K goes through S slots of 128 bytes (the
-// ring's slot layout) filled S - 1 slots ahead.
-template <int MJ, int NI, int S>
-struct SmallTile {
-  static constexpr int TM = 64 * MJ, TN = 64 * NI;
-  static constexpr int kSlotBytes = (TM + TN) * 128;
-  static constexpr int kLoadsA = TM / 32, kLoadsB = TN / 32;  // per wave and slot
-  static constexpr int kLoads = kLoadsA + kLoadsB;
-  static_assert(kSlotBytes >= TM * TN * 2 / S, "staging fits the slots");
-};
-
 template <int MJ, int NI, int S>
 struct SmallCtx {
   i32x4_t ra, rb;
@@ -1026,8 +1015,13 @@ __global__ __launch_bounds__(kThreads, WPC) void gemm_fp8_small(
     prm[T::TM + threadIdx.x] = psb;
     prm[T::TM + T::TN + threadIdx.x] = bf2f(pbias);
   }
-  __syncthreads();  // ... and every wave is done with the slots: the tile is staged in slot 0
-  uint16_t LDS_AS* ct = (uint16_t LDS_AS*)slot0;
+  __syncthreads();  // ... and every wave is done with the slots: the tile is staged in them
+  const auto row_of = [&](int r) {
+    if constexpr (T::kStageRows == T::TM)
+      return (uint16_t LDS_AS*)(sl[0] + T::stage_offset(r));
+    else
+      return (uint16_t LDS_AS*)((T::stage_slot(r) ? sl[1] : sl[0]) + T::stage_offset(r));
+  };
   const float LDS_AS* pl = (const float LDS_AS*)prm;
   const int h = c.lane >> 5;
 #pragma unroll
@@ -1044,13 +1038,12 @@ __global__ __launch_bounds__(kThreads, WPC) void gemm_fp8_small(
         float y[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) y[r] = acc[i][j][g * 4 + r] * (sam * sb[r]) + bv[r];
-        *(u32x2_t LDS_AS*)(ct + ml * T::TN + (((nl >> 2) ^ (ml & (T::TN / 4 - 1))) * 4)) =
+        *(u32x2_t LDS_AS*)(row_of(ml) + (((nl >> 2) ^ (ml & (T::TN / 4 - 1))) * 4)) =
             u32x2_t{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
       }
   }
   __syncthreads();
-  epi_rows<EPI, T::TM, T::TN>([&](int r) { return (const uint16_t LDS_AS*)(ct + r * T::TN); }, m0,
-                              n0, M, N, ep);
+  epi_rows<EPI, T::TM, T::TN>(row_of, m0, n0, M, N, ep);
 }
 
 // ---------------------------------------------------------------------------

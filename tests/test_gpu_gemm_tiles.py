@@ -20,6 +20,8 @@ _SHAPES = _STEPS + [
     (1152, 1536, 1536), (1025, 1400, 896),            # 64 x 128
     (2079, 1536, 1536), (1500, 1536, 1664),           # 128 x 128
     (2500, 1536, 4224), (3001, 1280, 4096),           # 128 x 256, long K
+    (2800, 1536, 4224), (4001, 1536, 4096),
+    *((4300, 1400, 128 * n) for n in range(1, 10)),   # 128 x 256, every remainder of its trips
     (2079, 4608, 512), (6200, 1536, 768),             # 192-row ring
     (7000, 1536, 4096), (12300, 1536, 512),           # ... long K, two rounds
 ]
