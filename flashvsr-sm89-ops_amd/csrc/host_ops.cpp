@@ -8,8 +8,10 @@
 //
 // Each function serves the plain case (exact tensors on one GPU, types and
 // layouts the kernels take as they are) and returns None for everything else,
-// including a refused launch: the Python caller then runs its general path,
-// which converts, checks and raises as documented there.
+// including a call the library refuses: the Python caller then runs its general
+// path, which converts, checks and raises as documented there.  A HIP error is
+// raised here: the library's status has taken it from the runtime, so a second
+// attempt would look clean, on work that may have failed.
 //
 // The C ABI functions are those of the library the Python side has loaded,
 // passed to bind() by address.
@@ -60,6 +62,14 @@ int dtype_code(const at::Tensor& t) {
   }
 }
 
+// What a call returns for a status other than FVSR_OK: None for one decided
+// before any launch, an exception for a HIP error (worded as the Python path's).
+PyObject* not_done(int rc, const char* what) {
+  if (rc != FVSR_EHIP) Py_RETURN_NONE;
+  PyErr_Format(PyExc_RuntimeError, "%s failed: HIP launch error (status %d)", what, rc);
+  return nullptr;
+}
+
 // quantize(x2, per_token, gelu) -> (codes, scale) or None
 PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -84,7 +94,7 @@ PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   rc = abi.quant_fp8_dt(x->data_ptr(), dt, M, K, x->stride(0), mode, gelu, q.data_ptr(),
                         (float*)s.data_ptr(), wn > 0 ? (float*)ws.data_ptr() : nullptr, wn, st);
   Py_END_ALLOW_THREADS
-  if (rc != FVSR_OK) Py_RETURN_NONE;
+  if (rc != FVSR_OK) return not_done(rc, gelu ? "fused_gelu_quant_fp8" : "quantize_fp8");
   PyObject* qo = THPVariable_Wrap(std::move(q));
   PyObject* so = qo ? THPVariable_Wrap(std::move(s)) : nullptr;
   PyObject* r = so ? PyTuple_Pack(2, qo, so) : nullptr;
@@ -135,7 +145,7 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
                     t[5] ? FVSR_EPI_ROWMAX : FVSR_EPI_BIAS,
                     t[5] ? (float*)t[5]->data_ptr() : nullptr, nullptr, nullptr, st);
   Py_END_ALLOW_THREADS
-  if (rc != FVSR_OK) Py_RETURN_NONE;
+  if (rc != FVSR_OK) return not_done(rc, "fp8_gemm");
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }

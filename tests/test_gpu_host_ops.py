@@ -116,6 +116,55 @@ def test_refusals_and_modes(general):
     _same(got, want)
 
 
+@pytest.fixture()
+def stub():
+    """Binds the native calls to a stand-in for the library's quantisation and
+    GEMM that launches nothing and returns the status it is given."""
+    import ctypes
+
+    from flashvsr_sm89_ops import _lib
+    host, L = _lib.host(), _lib.lib()
+    names = ("fvsr_quant_workspace_floats", "fvsr_quant_fp8_dt", "fvsr_fp8_gemm",
+             "fvsr_gemm_amax_parts")
+    real = [ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in names]
+    held = []
+
+    def bind(status):
+        calls = []
+        for i in (1, 2):
+            args, res = _lib._SIGS[names[i]]
+            held.append(ctypes.CFUNCTYPE(res, *args)(lambda *a: (calls.append(1), status)[1]))
+        addr = [ctypes.cast(f, ctypes.c_void_p).value for f in held[-2:]]
+        host.bind(real[0], *addr, real[3])
+        return calls
+    yield bind
+    host.bind(*real)
+
+
+def test_hip_errors_are_raised(stub):
+    """A HIP error is raised by the call that met it, as the general path does,
+    and the call is not made again; a refusal goes to the general path."""
+    import flashvsr_sm89_ops as fv
+    from flashvsr_sm89_ops import _lib
+    from flashvsr_sm89_ops.fp8_ffn import fused_gelu_quant_fp8
+    x = torch.randn(64, 256, device=DEV).bfloat16()
+    x8, s = fv.quantize_fp8(x, per_token=True)
+    w8, ws = fv.quantize_weight_fp8(torch.randn(96, 256, device=DEV).bfloat16(), per_channel=True)
+    y = fv.fp8_gemm(x8, s, w8, ws)
+    calls = [("quantize_fp8", lambda: fv.quantize_fp8(x, per_token=True), (x8, s)),
+             ("fused_gelu_quant_fp8", lambda: fused_gelu_quant_fp8(x, per_token=True), None),
+             ("fp8_gemm", lambda: fv.fp8_gemm(x8, s, w8, ws), y)]
+    for what, f, want in calls:
+        n = stub(_lib.FVSR_EHIP)
+        with pytest.raises(RuntimeError, match=f"{what} failed: HIP launch error .status -2"):
+            f()
+        assert len(n) == 1
+        for status in (_lib.FVSR_EINVAL, _lib.FVSR_EUNSUPPORTED, _lib.FVSR_EWORKSPACE):
+            n = stub(status)
+            got = f()
+            assert len(n) == 1 and (want is None or _same(got, want) is None)
+
+
 def test_streams(general):
     """The launch and the allocations follow torch's current stream."""
     import flashvsr_sm89_ops as fv
