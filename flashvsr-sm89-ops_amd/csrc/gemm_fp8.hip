@@ -1201,35 +1201,49 @@ struct Plan {
 
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// The kernel whose tiles finish first.  A CU works its tiles off one after the
-// other (or two side by side at half speed each), so a tile shape costs
-// rounds = ceil(tiles / CUs) times the clocks of one tile per 128 bytes of K:
-// what its LDS traffic takes at 128 bytes per clock (fragment reads plus the
-// loads' writes) up to 128 x 128, its MFMAs (64 clocks each) at 256 x 256.  The
-// two between are priced as measured: 192 rows at 1.17 of their MFMAs (1.22 at
-// long K, where the 256-row kernel prefetches into L2); 128 x 256 at 1.25 of
-// its LDS traffic, 1.07 at long K, where its start and epilogue weigh less.
-// Equal costs go to the larger tile.  Over 26 shapes (M 1300-15000, N 1536-8960,
-// K 1536 and 8960) the choice is within 4% of the fastest of the eight.
-// Where lines lie, both sides measured (us): M = 512 (N = K = 1536) 64 x 64
-// 5.5 against 64 x 128 7.1; M = 1152 8.5 / 8.2; M = 2079 128 x 128 11.3
-// against 64 x 128 11.7; M = 2800 ring 128 15.4 against 64 x 128 16.3; 12000
-// rows 192 against 256 32.7 / 35.4; 9000 rows 31.0 / 22.7; three rounds of 256
-// rows against five of 128 (4227 x 8960) 59.4 / 66.8.  At long K the 128 x 256
-// tile of gemm_fp8_small (three slots, 4000 rows 50.5) replaces the ring's
-// (two, 59.4); at K = 1536 its longer start costs more (16.5 / 15.3).
+// The kernel whose tiles finish first, by what its launch is measured to take:
+//   start + rounds * (epilogue + K / 128 * step),  rounds = ceil(tiles / CUs),
+// in ns (64-row tiles: times 1 + rounds / 800, they read the most operand bytes:
+// 56 rounds, 12996 x 8960 x 1536 with gate-add, 331 us against the ring's 307).
+// A CU works its tiles off one after the other (or two of the small ones side by
+// side at half speed each).  `step` is the K loop's: LDS traffic at 128 bytes per
+// clock (fragment reads plus the loads' writes) up to 128 x 128, MFMAs (64 clocks
+// each) at 256 x 256; deep_step the same at long K, where the 256-row kernel
+// prefetches into L2.  The epilogue's part is what short K turns on: the general
+// epilogue of kRing takes 12 us a tile for the bias and 32 for the gate-add
+// where kRing256's takes 11, and two 64 x 128 tiles to a CU hide most of theirs
+// under the other's K loop.
+//
+// The figures are a fit to 2895 measured calls, each by every kernel that could
+// take it (69 sets of K 128-8960, N 1280-8960 and epilogue, with whole and
+// partial column tiles, aligned and unaligned rows; M from 100 to 16896),
+// adjusted where the fit chose wrongly and checked on 2964 others: the choice is
+// on average 0.5% slower than the fastest, 3.5% at the 95th percentile, 20% at
+// most.  Priced by rounds * step alone it was 5.3%, 31% and 60%, and in places
+// slower than 256 x 256 everywhere had been (us, now / so / 256 x 256): K =
+// 1536, N = 1400: M = 12300 42.1 / 52.3 / 47.2; N = 4600: M = 4224 47.9 / 52.3 /
+// 47.9; K = 4096, N = 1280 with row maxima: M = 5014 30.8 / 34.5 / 31.6 (128-row
+// ring); gate-add, K = 1536, N = 1400: M = 7000 30.6 / 42.0 / 42.8.
 Plan plan_gemm(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int epilogue,
                bool direct) {
   struct Option {
     Path path;
-    int rows, cols, cost, deep_cost;  // deep: K >= kTouchMinK
+    int rows, cols, start;
+    int epilogue[3];  // bias, row maxima, gate-add
+    int unaligned;    // more per tile where the output's rows are not 16-byte chunks
+    int step, deep_step;  // deep: K >= kTouchMinK
   };
   static constexpr Option kOptions[] = {
-      {Path::kRing256, 256, 256, 2048, 2048}, {Path::kRing, 256, 256, 2048, 2048},
-      {Path::kRing192, 192, 256, 1800, 1880}, {Path::kRing128, 128, 256, 1440, 1440},
-      {Path::k128x256, 128, 256, 1440, 1230}, {Path::k128x128, 128, 128, 768, 768},
-      {Path::k64x128, 64, 128, 576, 576},     {Path::k64x64, 64, 64, 384, 384},
+      {Path::kRing256, 256, 256, -3220, {10640, 11180, 0}, 0, 845, 1050},
+      {Path::kRing, 256, 256, -3650, {12400, 22780, 32160}, 5360, 865, 995},
+      {Path::kRing192, 192, 256, -1280, {7800, 8100, 0}, 0, 730, 770},
+      {Path::kRing128, 128, 256, -600, {6280, 6600, 0}, 0, 550, 740},
+      {Path::k128x256, 128, 256, -2460, {12020, 15440, 18740}, 2760, 600, 540},
+      {Path::k128x128, 128, 128, 30, {6220, 7600, 9080}, 1680, 350, 390},
+      {Path::k64x128, 64, 128, 2860, {1360, 1640, 2320}, 780, 225, 245},
+      {Path::k64x64, 64, 64, 3100, {1000, 1500, 1640}, 680, 140, 150},
   };
+  static_assert(FVSR_EPI_BIAS == 0 && FVSR_EPI_ROWMAX == 1 && FVSR_EPI_GATE_ADD == 2, "");
   // Every row offset of either operand within 32 bits; the ring takes K in
   // pairs of 128 bytes, at least two of them.
   const bool small = K % 128 == 0 && K > 0 && K < 0x7fffffffLL &&
@@ -1237,21 +1251,24 @@ Plan plan_gemm(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int ep
   const bool ring = small && K % 256 == 0 && K >= 512;
   // The fast epilogue needs whole column tiles.
   const bool fast = ring && epilogue != FVSR_EPI_GATE_ADD && direct && N % BN == 0;
-  const bool deep = K >= kTouchMinK;
   const int64_t slots = persistent_slots();
   Plan best{Path::kGeneric, (unsigned)(cdiv(M, BM) * cdiv(N, BN))};
   int64_t best_cost = INT64_MAX;
   for (const Option& o : kOptions) {
-    bool ok = small;
-    if (o.path == Path::kRing) ok = ring && !fast;
-    if (o.path == Path::kRing256 || o.path == Path::kRing192) ok = fast;
-    if (o.path == Path::kRing128) ok = fast && !deep;
-    if (o.path == Path::k128x256) ok = small && (deep || !fast);
-    if (o.path == Path::k64x64) ok = small && epilogue != FVSR_EPI_ROWMAX;
+    bool ok = small, persistent = true;
+    switch (o.path) {
+      case Path::kRing: ok = ring && !fast; break;
+      case Path::kRing128: case Path::kRing192: case Path::kRing256: ok = fast; break;
+      case Path::k64x64: ok = small && epilogue != FVSR_EPI_ROWMAX; [[fallthrough]];
+      default: persistent = false;
+    }
     if (!ok) continue;
     const int64_t tiles = cdiv(M, o.rows) * cdiv(N, o.cols);
     if (tiles > 0x7fffffff) continue;
-    const int64_t rounds = cdiv(tiles, slots), cost = rounds * (deep ? o.deep_cost : o.cost);
+    const int64_t rounds = cdiv(tiles, slots);
+    const int64_t tile = o.epilogue[epilogue] + (direct ? 0 : o.unaligned) +
+                         K / 128 * (K >= kTouchMinK ? o.deep_step : o.step);
+    const int64_t cost = o.start + rounds * (tile + (o.rows == 64 ? tile * rounds / 800 : 0));
     if (cost >= best_cost) continue;
     best_cost = cost;
     // Persistent kernels: the fewest workgroups (a multiple of the 8 XCDs)
@@ -1260,8 +1277,6 @@ Plan plan_gemm(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int ep
     // tiles and fewer instead of 256 of 9 or 10; qkv 240, o and ffn2 200): the
     // critical path is unchanged and the idle CUs' power goes to the others'
     // clock (ffn0 216 -> 210 us, o 40.8 -> 39.7 us).
-    const bool persistent = o.path == Path::kRing || o.path == Path::kRing128 ||
-                            o.path == Path::kRing192 || o.path == Path::kRing256;
     best = {o.path, (unsigned)(persistent && tiles > slots ? 8 * cdiv(tiles, 8 * rounds) : tiles)};
   }
   return best;
@@ -1270,6 +1285,22 @@ Plan plan_gemm(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int ep
 }  // namespace
 
 extern "C" int64_t fvsr_gemm_amax_parts(int64_t N) { return (N + 127) / 128; }
+
+extern "C" const char* fvsr_gemm_tile(int64_t M, int64_t N, int64_t K, int epilogue, int rows16) {
+  if (M <= 0 || N <= 0 || K <= 0 || epilogue < FVSR_EPI_BIAS || epilogue > FVSR_EPI_GATE_ADD)
+    return "";
+  switch (plan_gemm(M, N, K, K, K, epilogue, rows16 != 0).path) {
+    case Path::k64x64: return "64x64";
+    case Path::k64x128: return "64x128";
+    case Path::k128x128: return "128x128";
+    case Path::k128x256: return "128x256";
+    case Path::kRing: return "ring";
+    case Path::kRing128: return "ring128";
+    case Path::kRing192: return "ring192";
+    case Path::kRing256: return K >= kTouchMinK ? "ring256 prefetching" : "ring256";
+    default: return "generic";
+  }
+}
 
 extern "C" int fvsr_fp8_gemm(const void* a, int64_t lda, const float* sa, int sa_mode,
                              const void* b, int64_t ldb, const float* sb, int sb_mode,

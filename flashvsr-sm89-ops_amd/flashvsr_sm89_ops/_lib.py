@@ -49,6 +49,7 @@ _SIGS = {
     "fvsr_fp8_gemm": ([_P, _I64, _P, _I, _P, _I64, _P, _I, _P, _P, _I64, _I64, _I64, _I64, _I,
                        _P, _P, _P, _P], _I),
     "fvsr_gemm_amax_parts": ([_I64], _I64),
+    "fvsr_gemm_tile": ([_I64, _I64, _I64, _I, _I], ctypes.c_char_p),
     "fvsr_ln_modulate": ([_P, _P, _P, _P, _I64, _I64, _I64, _F, _P, _P, _P], _I),
     "fvsr_gate_add": ([_P, _P, _P, _P, _I64, _I64, _I64, _P], _I),
     "fvsr_layer_norm": ([_P, _P, _P, _P, _I64, _I64, _F, _P, _P, _P], _I),

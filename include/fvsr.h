@@ -138,6 +138,15 @@ int fvsr_fp8_gemm(const void* a, int64_t lda, const float* sa, int sa_mode,
 /* Number of 128-column slabs FVSR_EPI_ROWMAX writes per row: ceil(N/128). */
 int64_t fvsr_gemm_amax_parts(int64_t N);
 
+/* Name of the kernel that fvsr_fp8_gemm runs on the current device (256 CUs
+ * without one) for packed operands (lda = ldb = K) of these sizes: the tile
+ * ("64x64" to "128x256"), "ring", "ring128", "ring192", "ring256", "ring256
+ * prefetching" or "generic"; "" for sizes or an epilogue it does not take.
+ * rows16: c is 16-byte aligned and ldc a multiple of 8, below 4 GB in all.
+ * A diagnostic: the results do not depend on it but for "generic", whose sums
+ * run in another order. */
+const char* fvsr_gemm_tile(int64_t M, int64_t N, int64_t K, int epilogue, int rows16);
+
 /*
  * LayerNorm (no affine) + modulate, reference fused_ln_modulate
  * (flashvsr_sm89_ops/fused_adaln.py:22-42,60-71): x bf16 [B,L,D];
