@@ -687,14 +687,24 @@ int64_t cu_count() {
 // is nearly as fast with one.  So it is whole units per CU that must come out
 // even: 108 units (a 24 x 24 tile) leave 148 CUs idle, 792 (66 query blocks)
 // give 24 CUs a fourth unit while the others wait.  The units past a multiple
-// of the CU count are cut into pieces, as many as two per CU take at once, at
-// least four of the maxk index entries each (a piece costs its start, ~6 us, and 130
-// KB of partials written and read).  Measured (one piece -> split, us):
-// 12 x 9 x 36 blocks 75 -> 42, 12 x 4 x 16 38 -> 21, 4 x 36 x 72 129 -> 75,
-// 12 x 66 x 66 379 -> 348, 12 x 66 x 198 941 -> 883, 12 x 17 x 68 132 -> 107.
-// Not split, since it measured the same or slower: a last round more than
-// three quarters full (39 x 12 units, 102.8 whole, 101.7 in two; 83 x 12, 603 /
-// 606) and calls of six rounds and more (132 x 12, 564 / 572).
+// of the CU count are cut into pieces, as many as two per CU take at once.  A
+// piece costs its start (~6 us) and 130 KB of partials written and read, the
+// combining launch 3 us more, so what the host knows of the call has to promise
+// more than that: at least four of the maxk index entries to a piece (eight, and
+// four pieces at most, behind whole units, whose end the pieces must meet), and
+// enough of them taken off the longest workgroup for the workgroups added (when
+// two pieces share a CU, more, since they share its speed too).
+// Measured, 60% of the blocks kept unless said (one piece -> split, us):
+// 12 x 9 x 36 blocks 72 -> 41, 12 x 4 x 16 38 -> 22, 4 x 36 x 72 126 -> 76,
+// 12 x 66 x 66, all kept, 478 -> 416, 12 x 66 x 198 862 -> 805, 12 x 17 x 68 120 ->
+// 96, 12 x 24 x 24 64 -> 58.
+// Not split, since it measured the same or slower: few entries (12 x 9 x 9, all
+// kept, 25 -> 27; 12 x 20 x 20 at 20% 27% slower, all kept 6%); a last round nearly
+// full, in the second round earlier, since its units find free slots (12 x 36 x
+// 144, all kept, 515 -> 546; 39 x 12 units 103 -> 102; 12 x 57 x 171 714 -> 659 is
+// split); calls of six rounds and more (132 x 12, 564 -> 572).
+// The host does not know the kept counts: where only a tenth of the blocks is
+// kept a split call of few units is slower than a whole one (12 x 9 x 18 17 -> 23).
 struct Split {
   int64_t whole, rest;
   int pieces;
@@ -705,9 +715,15 @@ Split plan_split(int64_t H, int64_t NQ, int64_t maxk) {
   const int64_t units = H * NQ, cus = cu_count();
   const Split plain{units, 0, 1};
   const int64_t rest = units % cus;
-  if (rest == 0 || units >= 6 * cus || (units > cus && 4 * rest > 3 * cus)) return plain;
-  const int64_t pieces = std::min({2 * cus / rest, maxk / 4, (int64_t)8});
-  return pieces > 1 ? Split{units - rest, rest, (int)pieces} : plain;
+  if (rest == 0 || units >= 6 * cus) return plain;
+  const bool tail = units > cus;
+  const int64_t pieces =
+      std::min({2 * cus / rest, maxk / (tail ? 8 : 4), (int64_t)(tail ? 4 : 8)});
+  if (pieces < 2) return plain;
+  if (tail && (units < 2 * cus ? 3 * rest > 2 * cus : 4 * rest > 3 * cus)) return plain;
+  const int64_t wgs = rest * pieces, saved = maxk - maxk / pieces;
+  if ((pieces == 2 && wgs > cus ? 24 : 40) * saved < wgs) return plain;
+  return Split{units - rest, rest, (int)pieces};
 }
 
 template <int QM, int KM, int MODE = kSparse>
