@@ -1,5 +1,5 @@
 """Build libfvsr.so (all HIP kernels + the C ABI) for gfx950 and the CPython
-extension _fvsr_host.so (csrc/host_ops.cpp), in-tree.
+extension _fvsr_host (csrc/host_ops.cpp), in-tree.
 
     python flashvsr-sm89-ops_amd/build.py [-j N]
 
@@ -8,8 +8,9 @@ linked into flashvsr_sm89_ops/libfvsr.so next to the Python package that
 loads it.  First, csrc/gelu_table_gen.c is compiled with gcc and run to
 write _build/gelu_table.inc (the bf16 GELU lookup table the quantisation
 kernels embed).  The extension is host code only, compiled with g++ against
-torch's headers; it gets the library's functions by address.  Flags: -O3 for gfx950 only, packed-fp32 instructions disabled
-(hipcc's host pass prints that it does not know the feature; harmless).
+torch's headers; it gets the library's functions by address.  Flags: -O3 for
+gfx950 only, packed-fp32 instructions disabled (hipcc's host pass prints that it
+does not know the feature; harmless).
 """
 import argparse
 import concurrent.futures as cf
@@ -18,6 +19,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -28,7 +30,9 @@ HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 
 CC = os.environ.get("CC", shutil.which("gcc") or "gcc")
 CXX = os.environ.get("CXX", shutil.which("g++") or "g++")
-HOST_LIB = os.path.join(HERE, "flashvsr_sm89_ops", "_fvsr_host.so")
+# Named for the Python it is built for: another one does not pick it up.
+HOST_LIB = os.path.join(HERE, "flashvsr_sm89_ops",
+                        "_fvsr_host" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 CFLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-I", OUT_DIR,
@@ -65,9 +69,7 @@ def _gelu_table() -> None:
 
 
 def _host_ext() -> None:
-    """Compile csrc/host_ops.cpp into _fvsr_host.so."""
-    import sysconfig
-
+    """Compile csrc/host_ops.cpp into HOST_LIB."""
     import torch
     t = os.path.dirname(torch.__file__)
     inc = [os.path.join(t, "include"), os.path.join(t, "include/torch/csrc/api/include"),
@@ -76,6 +78,7 @@ def _host_ext() -> None:
     tmp = HOST_LIB + ".tmp"
     cmd = [CXX, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
            "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f'-DFVSR_TORCH_VERSION="{torch.__version__}"',
            *(a for i in inc for a in ("-isystem", i)), os.path.join(CSRC, "host_ops.cpp"),
            "-o", tmp, "-L" + os.path.join(t, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu",
            "-ltorch_python"]

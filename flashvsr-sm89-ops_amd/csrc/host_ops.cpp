@@ -171,4 +171,9 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_fvsr_host", nullptr, -1, kMethod
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__fvsr_host() { return PyModule_Create(&kModule); }
+// torch_version: the torch whose headers this was compiled against.
+PyMODINIT_FUNC PyInit__fvsr_host() {
+  PyObject* m = PyModule_Create(&kModule);
+  if (m && PyModule_AddStringConstant(m, "torch_version", FVSR_TORCH_VERSION) < 0) Py_CLEAR(m);
+  return m;
+}

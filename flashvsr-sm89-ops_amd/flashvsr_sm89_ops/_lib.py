@@ -1,7 +1,8 @@
 """ctypes binding of libfvsr.so, the gfx950 kernels behind a C ABI.
 
 The library is loaded on first use.  There is no fallback: if the shared
-library is missing, or a tensor is not on a HIP device, the op raises.  All
+library is missing, or a tensor is not on a HIP device, the op raises (host(),
+which only saves host time, can be done without).  All
 launches go on torch's current stream of the tensor's device; the C side never
 allocates and never synchronises.
 """
@@ -10,6 +11,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 
 import torch
 
@@ -110,13 +112,21 @@ def lib():
     return _lib
 
 
+class _GeneralPath:
+    """Stands in for the extension where it cannot be used: every call is left
+    to the Python path, which reaches the same kernels through ctypes."""
+    quantize = gemm = staticmethod(lambda *args: None)
+
+
 _host = None
 
 
 def host():
     """The extension with the native host side of quantisation and GEMM
-    (csrc/host_ops.cpp), bound to the loaded library's functions; like the
-    library it must be built."""
+    (csrc/host_ops.cpp), bound to the loaded library's functions.  It only
+    saves host time, and unlike the library it is tied to the Python and torch
+    it was built with: where it does not load or was built with another torch, a
+    warning says why, once, and the calls take the Python path."""
     global _host
     if _host is None:
         L = lib()
@@ -124,13 +134,20 @@ def host():
             if _host is None:
                 try:
                     from . import _fvsr_host as h
+                    built = getattr(h, "torch_version", "of another version")
+                    if built != torch.__version__:
+                        raise ImportError(f"built with torch {built}, this is "
+                                          f"{torch.__version__}")
+                    h.bind(*(ctypes.cast(getattr(L, n), _P).value for n in (
+                        "fvsr_quant_workspace_floats", "fvsr_quant_fp8_dt", "fvsr_fp8_gemm",
+                        "fvsr_gemm_amax_parts")))
                 except ImportError as e:
-                    raise RuntimeError(
-                        "flashvsr_sm89_ops: _fvsr_host.so is not built. Build it with "
-                        "`python flashvsr-sm89-ops_amd/build.py`.") from e
-                h.bind(*(ctypes.cast(getattr(L, n), _P).value for n in (
-                    "fvsr_quant_workspace_floats", "fvsr_quant_fp8_dt", "fvsr_fp8_gemm",
-                    "fvsr_gemm_amax_parts")))
+                    warnings.warn(
+                        f"flashvsr_sm89_ops: the native host calls are off ({e}); FP8 "
+                        "quantisation and GEMM calls take several microseconds more of host "
+                        "time. Build them with `python flashvsr-sm89-ops_amd/build.py`.",
+                        RuntimeWarning, stacklevel=3)
+                    h = _GeneralPath
                 _host = h
     return _host
 
