@@ -79,7 +79,8 @@ PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
     Py_RETURN_NONE;
   const int dt = dtype_code(*x);
   if (dt < 0) Py_RETURN_NONE;
-  const bool per_token = PyObject_IsTrue(args[1]) == 1, gelu = PyObject_IsTrue(args[2]) == 1;
+  const int per_token = PyObject_IsTrue(args[1]), gelu = PyObject_IsTrue(args[2]);
+  if (per_token < 0 || gelu < 0) return nullptr;  // no truth value: its exception
   const int64_t M = x->size(0), K = x->size(1);
   const int mode = per_token ? FVSR_SCALE_ROW : FVSR_SCALE_TENSOR;
   at::Tensor q = at::empty({M, K}, x->options().dtype(at::kFloat8_e4m3fn));

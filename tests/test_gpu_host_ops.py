@@ -94,6 +94,10 @@ def test_refusals_and_modes(general):
                 call()
             kinds.append((e.type, str(e.value)))
         assert kinds[0] == kinds[1]
+    # a granularity without a truth value: the exception of asking for it
+    for call in (lambda f: f(), general):
+        with pytest.raises(RuntimeError, match="ambiguous"):
+            call(lambda: fv.quantize_fp8(torch.zeros(4, 8, device=DEV), torch.ones(2)))
     with pytest.raises(TypeError):
         fv.quantize_fp8(torch.zeros(4, 8, device=DEV, dtype=torch.int32))
     with pytest.raises(ValueError):
