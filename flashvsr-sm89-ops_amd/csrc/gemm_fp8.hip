@@ -936,16 +936,14 @@ __global__ __launch_bounds__(kThreads, WPC) void gemm_fp8_small(
     const uint8_t* __restrict__ A, int64_t lda, const uint8_t* __restrict__ B, int64_t ldb,
     int64_t M, int64_t N, int64_t K, EpiArgs ep) {
   using T = SmallTile<MJ, NI, S>;
-  static_assert(S >= 2 && S <= 6, "");
+  static_assert(S == 3 || S == 4, "");
   __shared__ __attribute__((aligned(1024))) uint8_t slot0[T::kSlotBytes];
   __shared__ __attribute__((aligned(1024))) uint8_t slot1[T::kSlotBytes];
-  __shared__ __attribute__((aligned(1024))) uint8_t slot2[S > 2 ? T::kSlotBytes : 16];
+  __shared__ __attribute__((aligned(1024))) uint8_t slot2[T::kSlotBytes];
   __shared__ __attribute__((aligned(1024))) uint8_t slot3[S > 3 ? T::kSlotBytes : 16];
-  __shared__ __attribute__((aligned(1024))) uint8_t slot4[S > 4 ? T::kSlotBytes : 16];
-  __shared__ __attribute__((aligned(1024))) uint8_t slot5[S > 5 ? T::kSlotBytes : 16];
   __shared__ __attribute__((aligned(16))) float prm[T::TM + 2 * T::TN];  // sa, sb, bias
-  uint8_t LDS_AS* sl[6] = {(uint8_t LDS_AS*)slot0, (uint8_t LDS_AS*)slot1, (uint8_t LDS_AS*)slot2,
-                           (uint8_t LDS_AS*)slot3, (uint8_t LDS_AS*)slot4, (uint8_t LDS_AS*)slot5};
+  uint8_t LDS_AS* sl[4] = {(uint8_t LDS_AS*)slot0, (uint8_t LDS_AS*)slot1, (uint8_t LDS_AS*)slot2,
+                           (uint8_t LDS_AS*)slot3};
   const int tiles_m = (int)((M + T::TM - 1) / T::TM), tiles_n = (int)((N + T::TN - 1) / T::TN);
   int tm, tn;
   map_tile(blockIdx.x, tiles_m, tiles_n, tm, tn);

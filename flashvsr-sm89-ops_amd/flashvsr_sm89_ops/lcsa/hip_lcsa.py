@@ -129,7 +129,7 @@ def block_sparse_attention_strided(q, k, v, keep, sm_scale=None, *, heads: int, 
         and 0 < NK <= _MASK_MAX
     if masked:
         _lib.require_gpu(keep)
-        maxk = max(NK, 1)
+        maxk = NK
     else:
         sel, cnt, maxk = block_index(keep) if index is None else index
     if H != heads:
