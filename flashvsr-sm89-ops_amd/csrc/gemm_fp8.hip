@@ -1149,18 +1149,22 @@ struct GemmArgs {
 };
 
 template <class Kernel>
-void start(Kernel kernel, unsigned grid, hipStream_t st, const GemmArgs& g) {
+int start(Kernel kernel, unsigned grid, hipStream_t st, const GemmArgs& g) {
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), 0, st, g.a, g.lda, g.b, g.ldb, g.M, g.N,
                      g.K, g.ep);
+  return fvsr_launch_status();
 }
 
 template <int EPI>
-void launch(Path path, unsigned grid, hipStream_t st, const GemmArgs& g) {
+int launch(Path path, unsigned grid, hipStream_t st, const GemmArgs& g) {
   switch (path) {
     case Path::kGeneric:
       return start(gemm_fp8_generic<EPI>, grid, st, g);
     case Path::kRing:
       return start(gemm_fp8_ring<EPI, false, 4>, grid, st, g);
+    case Path::k64x64:  // row maxima need 128-column tiles
+      if constexpr (EPI == FVSR_EPI_ROWMAX) break;
+      else return start(gemm_fp8_small<EPI, 1, 1, 4, 2>, grid, st, g);
     case Path::k64x128:
       return start(gemm_fp8_small<EPI, 1, 2, 3, 2>, grid, st, g);
     case Path::k128x128:
@@ -1170,15 +1174,14 @@ void launch(Path path, unsigned grid, hipStream_t st, const GemmArgs& g) {
     default:
       break;
   }
-  if constexpr (EPI != FVSR_EPI_ROWMAX) {  // row maxima need 128-column tiles
-    if (path == Path::k64x64) return start(gemm_fp8_small<EPI, 1, 1, 4, 2>, grid, st, g);
-  }
   if constexpr (EPI != FVSR_EPI_GATE_ADD) {  // gate-add keeps the general epilogue
     if (path == Path::kRing128) return start(gemm_fp8_ring<EPI, true, 2>, grid, st, g);
     if (path == Path::kRing192) return start(gemm_fp8_ring<EPI, true, 3>, grid, st, g);
-    if (g.K >= kTouchMinK) return start(gemm_fp8_ring<EPI, true, 4, true>, grid, st, g);
-    return start(gemm_fp8_ring<EPI, true, 4>, grid, st, g);
+    if (path == Path::kRing256)
+      return g.K >= kTouchMinK ? start(gemm_fp8_ring<EPI, true, 4, true>, grid, st, g)
+                               : start(gemm_fp8_ring<EPI, true, 4>, grid, st, g);
   }
+  return FVSR_EUNSUPPORTED;  // a plan that this epilogue has no kernel for
 }
 
 // Workgroups of the persistent kernel: one per CU, rounded down to a multiple
@@ -1329,14 +1332,10 @@ extern "C" int fvsr_fp8_gemm(const void* a, int64_t lda, const float* sa, int sa
   const Plan plan = plan_gemm(M, N, K, lda, ldb, epilogue, direct != 0);
   switch (epilogue) {
     case FVSR_EPI_BIAS:
-      launch<FVSR_EPI_BIAS>(plan.path, plan.grid, st, g);
-      break;
+      return launch<FVSR_EPI_BIAS>(plan.path, plan.grid, st, g);
     case FVSR_EPI_ROWMAX:
-      launch<FVSR_EPI_ROWMAX>(plan.path, plan.grid, st, g);
-      break;
+      return launch<FVSR_EPI_ROWMAX>(plan.path, plan.grid, st, g);
     default:
-      launch<FVSR_EPI_GATE_ADD>(plan.path, plan.grid, st, g);
-      break;
+      return launch<FVSR_EPI_GATE_ADD>(plan.path, plan.grid, st, g);
   }
-  return fvsr_launch_status();
 }
