@@ -56,3 +56,27 @@ def test_kernels_only_where_they_apply():
                     "ring192", "ring256", "ring256 prefetching"}
     for bad in ((0, 8, 128, 0), (8, 0, 128, 0), (8, 8, 0, 0), (8, 8, 128, 3), (8, 8, 128, -1)):
         assert _tile(*bad) == ""
+
+
+def test_shapes_of_the_gpu_tests_reach_every_kernel():
+    """The GPU tests' shapes run every kernel with each epilogue it has, on a
+    ragged last row tile, on a ragged last column tile where it takes one, and at
+    every remainder of the small tiles' trips."""
+    from test_gpu_gemm_tiles import _SHAPES
+    size = {"64x64": (64, 64, 4), "64x128": (64, 128, 6), "128x128": (128, 128, 4),
+            "128x256": (128, 256, 6), "ring": (256, 256, 1), "ring128": (128, 256, 1),
+            "ring192": (192, 256, 1), "ring256": (256, 256, 1),
+            "ring256 prefetching": (256, 256, 1)}
+    for epi in (BIAS, ROWMAX, GATE):
+        reached = {}
+        for shape in _SHAPES:
+            reached.setdefault(_tile(*shape, epi), []).append(shape)
+        want = set(size) - {"64x64"} if epi == ROWMAX else set(size)
+        if epi == GATE:
+            want -= {"ring128", "ring192", "ring256", "ring256 prefetching"}
+        assert set(reached) == want
+        for t, shapes in reached.items():
+            rows, cols, trip = size[t]
+            assert any(M % rows for M, _, _ in shapes)
+            assert any(N % cols for _, N, _ in shapes) or t[:5] in ("ring1", "ring2")
+            assert {K // 128 % trip for _, _, K in shapes} == set(range(trip)), (t, epi)

@@ -11,19 +11,25 @@ from test_gpu_ops import (DEV, _close_bf16, _gemm_inputs, codes_dev, dev_bf16, h
 
 pytestmark = pytest.mark.gpu
 
-# K steps of 128 around the pipelines' depths (2 to 4 slots, trips of 4 or 6),
-# on outputs of one or two ragged tiles.
-_STEPS = [(65, 72, 128 * n) for n in (1, 2, 3, 4, 5, 6, 7, 8, 9, 13)]
-_SHAPES = _STEPS + [
-    (1, 64, 256), (64, 64, 128), (63, 1000, 384),     # 64 x 64
-    (512, 1536, 1536), (129, 1544, 640),              # 64 x 64, 64 x 128
-    (1152, 1536, 1536), (1025, 1400, 896),            # 64 x 128
-    (2079, 1536, 1536), (1500, 1536, 1664),           # 128 x 128
-    (2500, 1536, 4224), (3001, 1280, 4096),           # 128 x 256, long K
-    (2800, 1536, 4224), (4001, 1536, 4096),
-    *((4300, 1400, 128 * n) for n in range(1, 10)),   # 128 x 256, every remainder of its trips
-    (2079, 4608, 512), (6200, 1536, 768),             # 192-row ring
-    (7000, 1536, 4096), (12300, 1536, 512),           # ... long K, two rounds
+# K steps of 128 around the pipelines' depths (trips of 4 or 6 steps).  Which
+# kernel a shape reaches depends on the epilogue (row maxima take 64 x 128 where
+# the others take 64 x 64); tests/test_gemm_plan.py checks that every kernel is
+# reached with each epilogue it has, at every remainder of its trips.
+_SHAPES = [(65, 72, 128 * n) for n in (1, 2, 3, 4, 5, 6, 7, 8, 9, 13)]
+_SHAPES += [(8200, 72, 128 * n) for n in (1, 2, 3, 4, 5, 6, 7)]       # 64 x 128
+_SHAPES += [(8200, 200, 128 * n) for n in (7, 8, 9, 14, 17, 18, 19, 20)]  # 128 x 128
+_SHAPES += [(10001, 520, 128 * n) for n in (5, 6, 7, 8, 9, 16, 17)]   # 128 x 256
+_SHAPES += [(4001, 1032, 128 * n) for n in (33, 34, 35, 36, 37, 38)]  # ... long K
+_SHAPES += [
+    (1, 64, 256), (64, 64, 128), (63, 1000, 384), (512, 1536, 1536),   # 64 x 64
+    (129, 1544, 640), (1152, 1536, 1536), (1025, 1400, 896),           # 64 x 128
+    (2079, 1536, 1536), (1500, 1536, 1664), (2500, 1536, 4224),        # 128 x 128
+    (3001, 1280, 4096), (2800, 1536, 4224), (4001, 1536, 4096),        # 128 x 256, long K
+    (4001, 2056, 512), (7001, 2056, 768), (8200, 1536, 1792),          # general ring
+    (5001, 2056, 4096), (4200, 4600, 1024),
+    (3301, 1280, 512), (3301, 1280, 4352),                             # 128-row ring
+    (3301, 2560, 512), (6200, 1536, 768), (7000, 1536, 4096), (12300, 1536, 512),  # 192-row
+    (8201, 1536, 768), (8449, 4608, 512), (8201, 1536, 4352),          # 256-row, prefetching
 ]
 
 

@@ -169,16 +169,34 @@ def test_hip_errors_are_raised(stub):
             assert len(n) == 1 and (want is None or _same(got, want) is None)
 
 
-def test_streams(general):
-    """The launch and the allocations follow torch's current stream."""
+def test_streams():
+    """The launches follow torch's current stream: their inputs are written on a
+    side stream behind some milliseconds of other work, other data each time,
+    and the work is still running when the calls have returned."""
     import flashvsr_sm89_ops as fv
     side = torch.cuda.Stream()
-    x = torch.randn(2048, 1536, device=DEV).bfloat16()
-    want = fv.quantize_fp8(x)
+    big = torch.randn(8192, 8192, device=DEV).bfloat16()
+    w8, ws = fv.quantize_weight_fp8(torch.randn(96, 1536, device=DEV).bfloat16(), per_channel=True)
+    xs = [torch.randn(2048, 1536, device=DEV).bfloat16() * (i + 1) for i in range(3)]
+    want = []
+    for x in xs:
+        x8, s = fv.quantize_fp8(x)
+        want.append((x8, s, fv.fp8_gemm(x8, s, w8, ws)))
+    y, z8, zs = torch.zeros_like(xs[0]), torch.zeros_like(want[0][0]), torch.ones_like(want[0][1])
+    big @ big
     torch.cuda.synchronize()
-    for _ in range(3):
+    for x, (x8, s, h) in zip(xs, want):
+        written = torch.cuda.Event()
         with torch.cuda.stream(side):
-            y = (x * 1.0).contiguous()      # on the side stream
+            for _ in range(8):
+                big @ big
+            y.copy_(x)
+            z8.copy_(x8)
+            zs.copy_(s)
+            written.record()
             got = fv.quantize_fp8(y)
+            g = fv.fp8_gemm(z8, zs, w8, ws)
+        assert not written.query(), "the inputs were there before the calls were made"
         side.synchronize()
-        _same(got, want)
+        _same(got, (x8, s))
+        _same(g, h)

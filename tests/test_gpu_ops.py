@@ -323,9 +323,9 @@ def test_gelu_tensor_quant_small_values(ops):
                                  (2100, 9000, 768), (600, 300, 1280), (1300, 4608, 1024),
                                  (700, 2048, 8960)])
 def test_fp8_gemm_ring_shapes(ops, MNK):
-    """The main-loop variants across K-step counts (persistent ring for K a
-    multiple of 256 and >= 512, register-staged loop otherwise), ragged M, N,
-    and more tiles than workgroups (several tiles per workgroup)."""
+    """Products across K-step counts (register-staged loop where K is no
+    multiple of 128, else a tile by size), ragged M, N, and more tiles than
+    workgroups (several tiles per workgroup)."""
     M, N, K = MNK
     a, b, sa, sb, bias = _gemm_inputs(M, N, K, seed=M * 3 + K)
     y = ops.fp8_gemm(codes_dev(a), torch.from_numpy(sa).to(DEV), codes_dev(b),
@@ -340,8 +340,9 @@ def test_fp8_gemm_direct_epilogue_rows_past_m(ops, MNK, epi):
     """Whole column tiles take the fast epilogue, whose stores of rows past M
     are dropped by the store descriptor's byte range: the output is a view of
     the first M rows of a larger buffer whose remaining rows must keep a
-    sentinel.  The first three shapes fit one round of 128-row tiles (the
-    128-row kernel), the last one does not (256-row tiles)."""
+    sentinel.  (4224, 1536, 1536) takes the 128-row ring and (2100, 8960, 512)
+    the 192-row one; the others take small tiles, whose epilogue checks the row.
+    The 256-row rings have their sentinel in test_gpu_gemm_tiles.py."""
     from flashvsr_sm89_ops import _lib
     M, N, K = MNK
     a, b, sa, sb, bias = _gemm_inputs(M, N, K, seed=11 * M + N)
