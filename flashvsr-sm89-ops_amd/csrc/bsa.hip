@@ -869,7 +869,8 @@ extern "C" int fvsr_bsa_fwd_window_ws(const void* q, const void* k, const void* 
   int rc = bsa_args_ok(q, k, v, o, q_tok_stride, q_head_stride, kv_tok_stride, kv_head_stride,
                        o_tok_stride, o_head_stride, sel, cnt, head_dim, H, NQ);
   if (rc != FVSR_OK) return rc;
-  // In-window byte offsets of the K/V stream are 32-bit: two frames of rows.
+  // Two frames of raster K/V rows within 4 GB: the limit the header states.  The
+  // stream itself reaches further (a lane's 32-bit offset spans four rows).
   const int64_t hw = height * width;
   if (kv_raster && 2 * hw * kv_tok_stride * 2 > 0xffffffffLL) return FVSR_EUNSUPPORTED;
   if (hw > 0x3fffffff) return FVSR_EUNSUPPORTED;

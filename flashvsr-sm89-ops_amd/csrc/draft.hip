@@ -121,10 +121,11 @@ __global__ __launch_bounds__(kPoolWaves * 64) void pool_kernel(
 // loads of 128 channels in flight together.  (Dot products by fp64 fmas with
 // the query values broadcast from LDS read the LDS 256 times per key block:
 // 11.5 us at 12 heads x 66 x 198 blocks against 8.4 here.)  Pass 2: wave w
-// takes row l0+w, its maximum, exponentials and sum by wave reductions, and writes the softmax as bf16 bits to attn[h][l0+w][:]
-// and, for the threshold search, the row's histogram of nonzero patterns by
-// high byte to hist[h][l0+w][0..127] (attn <= 1 or the NaN 0x7fc0, so the high
-// byte is below 128).
+// takes row l0+w, its maximum, exponentials and sum by wave reductions, and
+// writes the softmax as bf16 bits to attn[h][l0+w][:] and, for the threshold
+// search, the row's histogram of nonzero patterns by high byte to
+// hist[h][l0+w][0..127] (attn <= 1 or the NaN 0x7fc0, so the high byte is below
+// 128).
 constexpr int kRowsPerScoreWg = 4;
 constexpr int kKeyTiles = 4;  // 16-block key tiles per wave at a time
 
@@ -404,7 +405,7 @@ extern "C" int fvsr_draft_block_mask(const void* q, int64_t q_tok_stride, const 
       ((uintptr_t)workspace & 15))
     return FVSR_EUNSUPPORTED;
   if (workspace_floats < fvsr_draft_workspace_floats(H, D, NQ, NK)) return FVSR_EWORKSPACE;
-  // LDS holds 4 * NK floats; 2 * D + NK keeps the bound of an earlier layout.
+  // 2 * D + NK <= 3968 is the limit the header states; the LDS holds 4 * NK floats.
   if (2 * D + NK > 3968 || (NQ / q_temporal) * NK > 0x7fffffff || H * NQ > 0x7fffffff ||
       (NQ + NK) * ((H * D + 511) / 512) > 0x7fffffff)
     return FVSR_EUNSUPPORTED;

@@ -5,11 +5,11 @@ Reference path (flashvsr_sm89_ops/integrate.py:132-143,171):
 FP8 q projection, RMSNorm of q (no RoPE), dense attention of the 16896 video
 tokens over the prompt K/V cached by ``init_cross_kv``, and an FP8 o
 projection.  Here the dense attention runs on the attention kernel's dense
-mode (fvsr_attn_dense: every 128-key block, no block index, two query blocks
-per workgroup over one K/V stream), the LayerNorm emits the q projection's per-token e4m3
-codes in the same pass, and the residual add is a gate-add
-add with a unit gate (bf16(x + bf16(1 * y)) = bf16(x + y)), which inside a DiT
-block is fused with the AdaLN that follows it.
+mode (fvsr_attn_dense: every 128-key block, no block index, one or two query
+blocks per workgroup over one K/V stream), the LayerNorm emits the q projection's
+per-token e4m3 codes in the same pass, and the residual add is a gate-add with a
+unit gate (bf16(x + bf16(1 * y)) = bf16(x + y)), which inside a DiT block is
+fused with the AdaLN that follows it.
 """
 from __future__ import annotations
 

@@ -319,7 +319,7 @@ int64_t fvsr_draft_workspace_floats(int64_t H, int64_t D, int64_t NQ, int64_t NK
  * ids ascending, as in fvsr_block_index; the rest of the row is unspecified.
  * workspace: fvsr_draft_workspace_floats(H, D, NQ, NK).
  * Requires D % 8 == 0, token strides % 8 == 0, 16-byte aligned q and k, and
- * 2*D + NK <= 3968.
+ * 2*D + NK <= 3968 (FVSR_EUNSUPPORTED beyond).
  */
 int fvsr_draft_block_mask(const void* q, int64_t q_tok_stride, const int32_t* q_map,
                           const void* k, int64_t k_tok_stride, const int32_t* k_map, int64_t H,
@@ -362,7 +362,9 @@ int fvsr_bsa_fwd(const void* q, const void* k, const void* v, void* o, int64_t q
  * No map is read: token rows are computed, so the first K/V loads of a block
  * wait on no other load.  Requires frames % 2 == 0, height % 8 == 0,
  * width % 8 == 0, frames*height*width == NQ*128, plus fvsr_bsa_fwd's
- * requirements.
+ * requirements; with kv_raster = 1 also two frames of K/V rows within 4 GB
+ * (2 * height * width * kv_tok_stride elements of 2 bytes; FVSR_EUNSUPPORTED
+ * beyond).
  */
 int fvsr_bsa_fwd_window(const void* q, const void* k, const void* v, void* o,
                         int64_t q_tok_stride, int64_t q_head_stride, int64_t kv_tok_stride,
@@ -381,7 +383,13 @@ int fvsr_bsa_fwd_window(const void* q, const void* k, const void* v, void* o,
  *   workspace   16-byte aligned, at least that many floats (FVSR_EWORKSPACE
  *               otherwise), used until the call's kernels have run; NULL: no
  *               unit is split, exactly the call without _ws
- * Splitting changes the order of the softmax sums, not their precision.
+ * Splitting changes the order of the softmax sums, not their precision: a row's
+ * P is rounded to bf16 against its own piece's running maximum, and the pieces
+ * are added in fp32.  A row's bits therefore depend on what decides the split:
+ * H, NQ, maxk and the device's CU count (of the kept counts only its own, which
+ * cuts its list).  One mask through indexes of different maxk (build_csr's trimmed
+ * rows, fvsr_block_index's untrimmed ones), or one row in calls of different H or
+ * NQ, may differ in the last bits of bf16.  Equal calls give equal bits.
  */
 int64_t fvsr_bsa_workspace_floats(int64_t H, int64_t NQ, int64_t maxk);
 int fvsr_bsa_fwd_ws(const void* q, const void* k, const void* v, void* o, int64_t q_tok_stride,
@@ -412,8 +420,10 @@ int fvsr_bsa_fwd_window_ws(const void* q, const void* k, const void* v, void* o,
  * block, for the cross-attention's softmax(Q K^T * sm_scale) V over the
  * prompt K/V cached by init_cross_kv (integrate.py:132-143; upstream
  * self.attn(q, cache_k, cache_v)).  NQ*128 query tokens, NK*128 key tokens,
- * strides as in fvsr_bsa_fwd, no block index and no token map.  One
- * workgroup of 8 waves takes two query blocks over one K/V stream.
+ * strides as in fvsr_bsa_fwd, no block index and no token map.  A
+ * workgroup of 8 waves takes two query blocks over one K/V stream, or one of 4
+ * waves a single block where the pairs would leave CUs idle or the K/V rows lie
+ * more than 1.4 GB apart; the same bits.
  */
 int fvsr_attn_dense(const void* q, const void* k, const void* v, void* o, int64_t q_tok_stride,
                     int64_t q_head_stride, int64_t kv_tok_stride, int64_t kv_head_stride,
