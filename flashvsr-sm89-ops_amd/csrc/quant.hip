@@ -529,9 +529,16 @@ int partial_floats(int64_t rows) {
 }
 
 // Workgroups of the tensor-mode passes, one partial maximum each (at most
-// partial_floats): every wave the same number of rows but the last ones (8448
+// partial_floats).  As many as there may be, except for long rows read in
+// chunks: there every wave gets the same number of rows but the last ones (8448
 // rows: 704 workgroups of 3 rows a wave, not 1024 of which 64 have a third).
-int partial_blocks(int64_t rows) {
+// Both passes, us, 1024 / even: 4224 x 8960 36.4 / 33.0, 8448 x 8960 61.2 / 57.9,
+// 8448 x 4608 33.3 / 32.3; but 8448 x 1536 11.3 / 12.1, 4701 x 2048 15% and 4224 x
+// 3072 9% slower, and element loads 8448 x 8960 fp32 424 / 448: short rows want
+// the waves.
+constexpr int64_t kLongRow = 4608;
+int partial_blocks(int64_t rows, bool even) {
+  if (!even) return partial_floats(rows);
   const int64_t b = (rows + kWaves - 1) / kWaves, per = (b + kMaxPartials - 1) / kMaxPartials;
   return b > 0 ? (int)((b + per - 1) / per) : 1;
 }
@@ -596,7 +603,7 @@ void launch_gelu_tensor_codes(const uint16_t* x, int64_t rows, int64_t cols, int
 template <bool GELU>
 int launch_tensor_scalar(const void* x, int dt, int64_t rows, int64_t cols, int64_t ld,
                          uint8_t* q, float* s, float* ws, hipStream_t st) {
-  const int P = partial_blocks(rows);
+  const int P = partial_blocks(rows, false);
   hipLaunchKernelGGL((amax_partial<GELU, false>), dim3(P), dim3(kThreads), 0, st, x, dt, rows,
                      cols, ld, ws);
   hipLaunchKernelGGL((quant_tensor<GELU, false>), dim3(P), dim3(kThreads), 0, st, x, dt, rows,
@@ -607,8 +614,8 @@ int launch_tensor_scalar(const void* x, int dt, int64_t rows, int64_t cols, int6
 template <bool GELU>
 int launch_tensor(const uint16_t* x, int64_t rows, int64_t cols, int64_t ld, uint8_t* q,
                   float* s, float* ws, hipStream_t st) {
-  const int P = partial_blocks(rows);
   const bool vec = (cols % 8 == 0) && (ld % 8 == 0) && aligned16(x) && aligned16(q);
+  const int P = partial_blocks(rows, vec && !GELU && cols >= kLongRow);
   if (vec && GELU && (cols / 8 + 63) / 64 <= 18) {
     // both passes by table; the grid is persistent, one partial per workgroup
     const int64_t g = std::min(table_blocks(rows), (int64_t)P);
@@ -663,7 +670,7 @@ extern "C" int fvsr_gelu_quant_fp8_tensor(const void* h, int64_t rows, int64_t c
   if (rows < 0 || cols < 0 || nparts <= 0) return FVSR_EINVAL;
   if (rows == 0 || cols == 0) return FVSR_OK;
   if (!h || !codes || !scale_out || !hmax_part) return FVSR_EINVAL;
-  const int P = partial_blocks(rows);
+  const int P = partial_blocks(rows, cols >= kLongRow);
   if (!workspace || workspace_floats < 2 * partial_floats(rows)) return FVSR_EWORKSPACE;
   hipStream_t st = (hipStream_t)stream;
   const uint16_t* hp = (const uint16_t*)h;
@@ -699,7 +706,7 @@ extern "C" int fvsr_quant_weight_fp8_dt(const void* w, int w_dtype, int64_t n, i
                        dim3(kThreads), 0, st, w, w_dtype, n, k, qp, scale_out);
     return fvsr_launch_status();
   }
-  const int P = partial_blocks(n);
+  const int P = partial_blocks(n, false);
   if (!workspace || workspace_floats < partial_floats(n)) return FVSR_EWORKSPACE;
   hipLaunchKernelGGL((amax_partial<false, false>), dim3(P), dim3(kThreads), 0, st, w, w_dtype, n,
                      k, k, workspace);

@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("gelu", [False, True])
 @pytest.mark.parametrize("rows,cols", [(1, 8), (3, 1536), (255, 64), (256, 520), (257, 1544),
                                        (4095, 16), (4096, 24), (4097, 16), (8193, 40),
-                                       (12289, 8), (300, 9224)])
+                                       (12289, 8), (300, 9224), (1025, 512), (70, 1024),
+                                       (70, 1032), (4100, 4600), (4100, 4608)])
 def test_tensor_mode_grids(rows, cols, gelu):
     import flashvsr_sm89_ops as ops
     from flashvsr_sm89_ops.fp8_ffn import fused_gelu_quant_fp8
