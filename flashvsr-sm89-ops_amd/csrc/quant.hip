@@ -57,13 +57,13 @@ FVSR_DEV float qscale(float amax) { return fmaxf(amax, 1e-12f) / 448.0f; }
 // The residual's copy of s, kept finite (s = inf when amax = inf).
 FVSR_DEV float qscale_fin(float s) { return fminf(s, 3.40282347e38f); }
 
-// Maximum over the workgroup's W waves of non-negative values (every load in
-// flight, into LDS too, has landed for all of them afterwards).
-template <int W>
+// Maximum over the workgroup's W waves of non-negative values.  LDS_LOADS: this
+// wave's direct loads into LDS have landed first, so the barrier covers them too.
+template <int W, bool LDS_LOADS = false>
 FVSR_DEV float block_max(float m, float* red) {
   m = wave_max_abs(m);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-  __builtin_amdgcn_s_waitcnt(0);
+  if (LDS_LOADS) __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   float r = red[0];
 #pragma unroll
@@ -72,11 +72,13 @@ FVSR_DEV float block_max(float m, float* red) {
 }
 
 // This thread's share (of T threads) of the largest of n partial maxima, 1 <= n
-// <= kMaxPartials: the loads are unconditional (past the end the last value
-// again), so they cost one memory latency together and not one each (the four
-// small passes of the per-tensor FFN at 8448 rows: 24 -> 20 us).
+// <= kMaxPartials; `none` (no larger than any of them) where it has none.  Up to
+// T of them take one load per thread.  More: the loads are unconditional (past
+// the end the last value again), so they cost one memory latency together and not
+// one each (the four small passes of the per-tensor FFN at 8448 rows: 24 -> 20 us).
 template <int T>
-FVSR_DEV float max_partials(const float* __restrict__ part, int n) {
+FVSR_DEV float max_partials(const float* __restrict__ part, int n, float none) {
+  if (n <= T) return (int)threadIdx.x < n ? part[threadIdx.x] : none;
   constexpr int U = (kMaxPartials + T - 1) / T;
   float v[U];
 #pragma unroll
@@ -102,7 +104,7 @@ FVSR_DEV void for_chunks(const uint16_t* row, int64_t n, int lane, const F& f) {
     for (int u = 0; u < U; ++u) f(c0 + 64 * u, v[u]);
   }
 }
-constexpr int kChunkLoads = 3;  // a 1536-column row in one go
+constexpr int kChunkLoads = 3;  // a 1536-column row in one go; shorter rows take what they hold
 
 // ---------------------------------------------------------------------------
 // Row mode, register resident: cols % 8 == 0, cols <= 512*VPL, 16-byte rows.
@@ -285,7 +287,7 @@ __global__ __launch_bounds__(kTabWaves * 64) void quant_tensor_gelu_table(
   __shared__ __attribute__((aligned(16))) uint16_t tab[65536];
   __shared__ float red[kTabWaves];
   load_table<kTabWaves>(tab);
-  const float amax = block_max<kTabWaves>(max_partials<kTabWaves * 64>(part, nparts), red);
+  const float amax = block_max<kTabWaves, true>(max_partials<kTabWaves * 64>(part, nparts, 0.0f), red);
   const float s = qscale(amax), r = 1.0f / s, sc = qscale_fin(s);
   if (blockIdx.x == 0 && threadIdx.x == 0) scale_out[0] = act_scale(amax);
   const int nchunk = (int)(cols >> 3);
@@ -367,8 +369,9 @@ __global__ __launch_bounds__(kThreads) void quant_rows_generic(
 // Tensor mode.
 // ---------------------------------------------------------------------------
 // Partial |x| maxima: workgroup b covers rows b, b+G, ... (one wave per row).
-// VEC: bf16 rows in 16-byte chunks; otherwise element loads of type dt.
-template <bool GELU, bool VEC>
+// VEC: bf16 rows in 16-byte chunks, U of them per lane at a time; otherwise
+// element loads of type dt.
+template <bool GELU, bool VEC, int U = kChunkLoads>
 __global__ __launch_bounds__(kThreads) void amax_partial(
     const void* __restrict__ x, int dt, int64_t rows, int64_t cols, int64_t ld,
     float* __restrict__ part) {
@@ -379,7 +382,7 @@ __global__ __launch_bounds__(kThreads) void amax_partial(
        row += (int64_t)gridDim.x * kWaves) {
     if (VEC) {
       // a repeated chunk changes no maximum
-      for_chunks<kChunkLoads>((const uint16_t*)x + row * ld, cols >> 3, lane,
+      for_chunks<U>((const uint16_t*)x + row * ld, cols >> 3, lane,
                               [&](int64_t, const u32x4_t& v) {
                                 m = fmaxf(m, chunk_absmax(GELU ? gelu_chunk(v) : v));
                               });
@@ -412,15 +415,15 @@ __global__ __launch_bounds__(kThreads) void max_reduce_signed(const float* __res
 }
 
 // Codes against the tensor's scale (the partial maxima reduced again by every
-// workgroup).  VEC: bf16 rows in 16-byte chunks; otherwise element loads of
-// type dt and the IEEE quotient.
-template <bool GELU, bool VEC>
+// workgroup).  VEC: bf16 rows in 16-byte chunks, U of them per lane at a time;
+// otherwise element loads of type dt and the IEEE quotient.
+template <bool GELU, bool VEC, int U = kChunkLoads>
 __global__ __launch_bounds__(kThreads) void quant_tensor(
     const void* __restrict__ x, int dt, int64_t rows, int64_t cols, int64_t ld,
     const float* __restrict__ part, int nparts, uint8_t* __restrict__ codes,
     float* __restrict__ scale_out) {
   __shared__ float red[kWaves];
-  const float amax = block_max<kWaves>(max_partials<kThreads>(part, nparts), red);
+  const float amax = block_max<kWaves>(max_partials<kThreads>(part, nparts, 0.0f), red);
   const float s = qscale(amax), r = 1.0f / s;
   if (blockIdx.x == 0 && threadIdx.x == 0) scale_out[0] = act_scale(amax);
   const int lane = threadIdx.x & 63;
@@ -429,7 +432,7 @@ __global__ __launch_bounds__(kThreads) void quant_tensor(
     uint8_t* qr = codes + row * cols;
     if (VEC) {
       const int64_t n = cols >> 3;
-      for_chunks<kChunkLoads>((const uint16_t*)x + row * ld, n, lane,
+      for_chunks<U>((const uint16_t*)x + row * ld, n, lane,
                               [&](int64_t c, const u32x4_t& v) {
                                 if (c < n)
                                   *(u32x2_t*)(qr + c * 8) = chunk_codes_fma(
@@ -452,7 +455,7 @@ __global__ __launch_bounds__(kThreads) void gelu_amax_from_hmax(
     const uint16_t* __restrict__ h, int64_t rows, int64_t cols, const float* __restrict__ hpart,
     int nh, float* __restrict__ gpart) {
   __shared__ float red[kWaves];
-  float hm = wave_max(max_partials<kThreads>(hpart, nh));
+  float hm = wave_max(max_partials<kThreads>(hpart, nh, -__builtin_huge_valf()));
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = hm;
   __syncthreads();
   hm = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
@@ -511,7 +514,7 @@ __global__ __launch_bounds__(kThreads) void quant_weight_tensor(
     const void* __restrict__ w, int dt, int64_t n, int64_t k, const float* __restrict__ part,
     int nparts, uint8_t* __restrict__ codes, float* __restrict__ scale_out) {
   __shared__ float red[kWaves];
-  const float s = weight_scale(block_max<kWaves>(max_partials<kThreads>(part, nparts), red), dt);
+  const float s = weight_scale(block_max<kWaves>(max_partials<kThreads>(part, nparts, 0.0f), red), dt);
   if (blockIdx.x == 0 && threadIdx.x == 0) scale_out[0] = s;
   const int64_t total = n * k;
   for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < total;
@@ -628,10 +631,17 @@ int launch_tensor(const uint16_t* x, int64_t rows, int64_t cols, int64_t ld, uin
                        FVSR_DT_BF16, rows, cols, ld, ws);
     launch_gelu_tensor_codes(x, rows, cols, ld, ws, P, q, s, st);
   } else if (vec) {
-    hipLaunchKernelGGL((amax_partial<GELU, true>), dim3(P), dim3(kThreads), 0, st, x,
-                       FVSR_DT_BF16, rows, cols, ld, ws);
-    hipLaunchKernelGGL((quant_tensor<GELU, true>), dim3(P), dim3(kThreads), 0, st, x,
-                       FVSR_DT_BF16, rows, cols, ld, ws, P, q, s);
+    // Three loads of which a short row holds one or two cost 5-9% there (both
+    // passes at 512 rows x 64 5.8 us, 5.4 with one; 16384 x 512 10.9, 9.0).
+    const auto run = [&](auto amax, auto quant) {
+      hipLaunchKernelGGL(amax, dim3(P), dim3(kThreads), 0, st, x, FVSR_DT_BF16, rows, cols, ld,
+                         ws);
+      hipLaunchKernelGGL(quant, dim3(P), dim3(kThreads), 0, st, x, FVSR_DT_BF16, rows, cols, ld,
+                         ws, P, q, s);
+    };
+    if (cols <= 512) run(amax_partial<false, true, 1>, quant_tensor<false, true, 1>);
+    else if (cols <= 1024) run(amax_partial<false, true, 2>, quant_tensor<false, true, 2>);
+    else run(amax_partial<false, true>, quant_tensor<false, true>);
   } else {
     return launch_tensor_scalar<GELU>(x, FVSR_DT_BF16, rows, cols, ld, q, s, ws, st);
   }
